@@ -25,8 +25,9 @@
 //    while ragged rows read just their own keys.  The splits' partials are merged by a second launch or by the
 //    last split to finish (ticket per (row, head)); a row with one split writes its output directly.
 // bf16 with head_dim a multiple of 128 runs on MFMA with every K/V element loaded straight into the operand layout
-// (128-bit loads, no LDS); fp32, or bf16 with another head_dim, runs a vector-ALU wave with fp32 products (the
-// reference's IEEE path for fp32 agreement checks).  The beams' attention (context by these kernels, generated
+// (128-bit loads, no LDS); fp32 at head dims 128, 256 and 512 runs the same shape on the fp32 MFMA instruction
+// (verify_attn_f32_kernel); other head dims, and rows not 16-byte aligned, run a vector-ALU wave with fp32 products.
+// The beams' attention (context by these kernels, generated
 // keys through pointers) is at the end of the file.
 #include <math.h>
 
@@ -169,10 +170,9 @@ __device__ __forceinline__ int merge_slot(const AttnArgs& a, int nact, int q) {
 // Log-sum-exp merge of the partials of (row b, head h) by one wave (the merge launch, after the split kernel);
 // writes the output.
 template <typename OutT>
-__device__ void merge_splits(const AttnArgs& a, int b, int h, int nact) {
+__device__ void merge_splits(const AttnArgs& a, int b, int h, int nact, int64_t split0) {
   const int lane = lane_id();
   const int nq = nact + (a.gen_split >= 0 ? 1 : 0);
-  const int64_t split0 = ((int64_t)b * a.H + h) * a.splits;
   OutT* out = reinterpret_cast<OutT*>(a.out);
   auto get = [](const float* p) { return *p; };
   for (int t = 0; t < a.T; ++t) {
@@ -600,11 +600,12 @@ __global__ __launch_bounds__(256) void beam_gen_list_kernel(GenListArgs a) {
   if (tid == 0) a.count[grp] = total;
 }
 
+// The deal: wk[b] workgroups of each head for row b (LDS; the caller's rows <= blockDim.x).
 template <bool GEN = false>
-__device__ BalancedSplit balanced_split(const AttnArgs& a, int j, int* gl = nullptr) {
-  __shared__ int nt[kBalancedMaxRows], wk[kBalancedMaxRows], rem[kBalancedMaxRows];
+__device__ __forceinline__ void balanced_deal(const AttnArgs& a, int* wk, int* gl = nullptr) {
+  __shared__ int nt[kBalancedMaxRows], rem[kBalancedMaxRows];
   __shared__ int s_total, s_given;
-  const int tid = threadIdx.x, rows = a.rows, budget = a.splits;  // the launcher ensures rows <= blockDim.x
+  const int tid = threadIdx.x, rows = a.rows, budget = a.splits;
   if (tid < rows) {
     int n = (int)((split_range(a, tid, 0).total + 31) >> 5);
     if constexpr (GEN) {
@@ -648,9 +649,16 @@ __device__ BalancedSplit balanced_split(const AttnArgs& a, int j, int* gl = null
   __syncthreads();
   if (tid < rows) wk[tid] += extra;
   __syncthreads();
+}
+
+// Workgroup j of a head: its row and split.
+template <bool GEN = false>
+__device__ BalancedSplit balanced_split(const AttnArgs& a, int j, int* gl = nullptr) {
+  __shared__ int wk[kBalancedMaxRows];
+  balanced_deal<GEN>(a, wk, gl);
   BalancedSplit out{-1, 0, 1, 0};
   int first = 0;
-  for (int b = 0; b < rows; ++b) {
+  for (int b = 0; b < a.rows; ++b) {
     if (j < first + wk[b]) {
       out = BalancedSplit{b, j - first, wk[b], first};
       break;
@@ -658,6 +666,15 @@ __device__ BalancedSplit balanced_split(const AttnArgs& a, int j, int* gl = null
     first += wk[b];
   }
   return out;
+}
+
+// Row b's splits of each head: their number and the first one's workgroup.
+__device__ __forceinline__ BalancedSplit balanced_row(const AttnArgs& a, int b) {
+  __shared__ int wk[kBalancedMaxRows];
+  balanced_deal<false>(a, wk);
+  int first = 0;
+  for (int o = 0; o < b; ++o) first += wk[o];
+  return BalancedSplit{b, 0, wk[b], first};
 }
 
 // Split-K for head dims past 128 (256, 512): one workgroup of D/128 waves per (split, head, row), wave w holding
@@ -874,6 +891,207 @@ __global__ __launch_bounds__(64 * (D / 128), G == 1 ? 2 : 1) void verify_attn_sl
   // workgroup slots, one per (group, head).
   const int64_t gen_slot = a.balanced ? (int64_t)a.H * a.splits + (int64_t)b * a.H + h : -1;
   merge_splits_fast<uint16_t>(a, b, h, r.nact, sl * 128, 128, slot0, gen_slot);
+  if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ---------------------------------------------------------------------------------------------- fp32 on MFMA
+
+// fp32 caches at head dims 128, 256 and 512 (16-byte aligned rows): the slice kernel's shape on
+// v_mfma_f32_16x16x4_f32, products and sums in fp32.  A workgroup of D/128 waves per split, wave w holding dimensions
+// 128w .. 128w + 127; a tile is 16 keys (16 KB of K and V per wave, two tiles in flight: the bytes and registers of
+// the bf16 kernel's 32-key tile).  HBM bounds it: the T <= 16 queries, padded to 16, share each read, and a tile's
+// products take 2048 clocks per SIMD where a CU's share of HBM delivers the tile's 64 KB (D = 512) in ~7000.
+// Layouts, lane (c = lane % 16, g = lane / 16), all from 16-byte loads with no permutes:
+//   S^T = K Q^T  step (j, e): A = K[key c][16j + 4g + e], B = Q[query c][16j + 4g + e]; lane (c, g) gets query c's
+//                scores of keys 4g + i;
+//   O = P V      step i: A = P[query c][key 4g + i] (the lane's own score i as a probability), B = V[key 4g + i][64b +
+//                4c + e], accumulator (b, e): rows 4g + r are queries, column c dimension 64b + 4c + e.
+// Measured, 8 rows x 8 heads x 512, one query, 750-2048 keys (426 MB a launch): 86 us with its merge, 4.9 TB/s, the
+// rate of a plain copy; the vector-ALU kernel below took 1415 us (301 GB/s: a key per lane, 4-byte loads 2 KB apart).
+// Against 64-bit results the error is 4e-7, the vector ALU's 9e-7.
+struct KVTileF32 {
+  f32x4_t k[8];     // key c, dimensions 16j + 4g ..
+  f32x4_t v[2][4];  // key 4g + i, dimensions 64b + 4c ..
+};
+
+// K rows past ``kmax`` and V rows at or past ``vstop`` (both relative to the tile) are read at the last valid row, as
+// in load_tile_clamped.  ``row``: bytes between key rows.
+__device__ __forceinline__ void load_tile_f32(KVTileF32& t, const char* kt, const char* vt, uint32_t row, int kmax,
+                                              int vstop, int c, int g) {
+  const uint32_t ko = (uint32_t)(c < kmax ? c : kmax) * row + g * 16;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) t.k[j] = *reinterpret_cast<const f32x4_t*>(kt + ko + j * 64);
+  int vmax = vstop - 1 < kmax ? vstop - 1 : kmax;
+  vmax = vmax > 0 ? vmax : 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int rv = 4 * g + i;
+    const uint32_t vo = (uint32_t)(rv < vmax ? rv : vmax) * row + c * 16;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) t.v[b][i] = *reinterpret_cast<const f32x4_t*>(vt + vo + b * 256);
+  }
+}
+
+template <int D>
+__global__ __launch_bounds__(64 * (D / 128), 2) void verify_attn_f32_kernel(AttnArgs a) {
+  constexpr int NSL = D / 128;
+  __shared__ f32x4_t sx[2][NSL][kWave];  // partial scores of a tile by slice, double-buffered
+  const int h = blockIdx.y;
+  int sp, b;
+  SplitRange r;
+  int64_t slot0;  // partial slot of the unit's first split
+  if (a.balanced) {
+    const BalancedSplit bs = balanced_split<false>(a, blockIdx.x);
+    if (bs.b < 0) return;  // uniform over the workgroup
+    b = bs.b;
+    sp = bs.k;
+    r = split_range(a, b, 0);
+    r.nact = bs.nact;
+    slot0 = (int64_t)h * a.splits + bs.first;
+  } else {
+    sp = blockIdx.x;
+    b = blockIdx.z;
+    r = split_range(a, b, sp);
+    if (sp >= r.nact) return;  // uniform over the workgroup
+    slot0 = ((int64_t)b * a.H + h) * a.splits;
+  }
+  const int lane = lane_id(), sl = threadIdx.x / kWave, c = lane & 15, g = lane >> 4;
+  const int T = a.T;
+  f32x4_t q[8];
+  {
+    const float* qrow = reinterpret_cast<const float*>(a.q) + ((int64_t)(b * T + (c < T ? c : 0)) * a.H + h) * D +
+                        sl * 128 + g * 4;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      q[j] = c < T ? *reinterpret_cast<const f32x4_t*>(qrow + j * 16) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  SoftmaxState st{-INFINITY, -INFINITY, 0.f};
+  f32x4_t o[8];
+#pragma unroll
+  for (int nb = 0; nb < 8; ++nb) o[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int64_t own = r.n + (a.causal ? c : 0);
+  const int lim = (int)(own < r.total ? own : r.total);
+
+  // The split's tiles: sp, sp + nact, ... of the row's 16-key tiles.
+  const int64_t row_tiles = (r.total + 15) >> 4;
+  const int64_t ntot = sp < row_tiles ? (row_tiles - sp + r.nact - 1) / r.nact : 0;
+  const uint32_t row = (uint32_t)a.s_pos * 4u;
+  const char* kt = reinterpret_cast<const char*>(a.k) + (b * a.s_row + h * a.s_head + sl * 128) * 4;
+  const char* vt = reinterpret_cast<const char*>(a.v) + (b * a.s_row + h * a.s_head + sl * 128) * 4;
+  const int64_t last_key = a.cache_len - 1;
+  const float c_scale = a.scale_log2;
+  auto load_k = [&](KVTileF32& t, int64_t k) {
+    const int64_t kb = (sp + k * r.nact) * 16;
+    const int64_t kmax = last_key - kb, vstop = r.total - kb, off = kb * row;
+    load_tile_f32(t, kt + off, vt + off, row, kmax < 15 ? (int)kmax : 15, vstop < 16 ? (int)vstop : 16, c, g);
+  };
+  auto attend_k = [&](const KVTileF32& t, int64_t k) {
+    f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(t.k[j][e], q[j][e], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(t.k[j + 1][e], q[j + 1][e], s1, 0, 0, 0);
+      }
+    }
+    f32x4_t s = s0 + s1;
+    if constexpr (NSL > 1) {
+      sx[k & 1][sl][lane] = s;
+      lds_barrier();
+      s = sx[k & 1][0][lane];
+#pragma unroll
+      for (int w = 1; w < NSL; ++w) s += sx[k & 1][w][lane];
+    }
+    const int key0 = (int)((sp + k * r.nact) * 16) + 4 * g;
+    bool over = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s[i] = key0 + i < lim ? s[i] : -INFINITY;
+      over |= s[i] > st.thr;
+    }
+    if (__any(over)) {
+      float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+      mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+      const float m_new = fmaxf(st.m_ref, mx * c_scale);
+      rescale<8>(st.m_ref, m_new == -INFINITY ? 0.f : m_new, st.l_run, o, g);
+      st.m_ref = m_new;
+      st.thr = m_new == -INFINITY ? -INFINITY : (m_new + kLazyLog2) / c_scale;
+    }
+    const float m_use = st.m_ref == -INFINITY ? 0.f : st.m_ref;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c_scale, -m_use));
+      st.l_run += p;
+#pragma unroll
+      for (int nb = 0; nb < 8; ++nb)
+        o[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, t.v[nb >> 2][i][nb & 3], o[nb], 0, 0, 0);
+    }
+  };
+  // The buffer written for tile k was last read for tile k - 2, before every wave passed tile k - 1's barrier.
+  if (ntot > 0) {
+    KVTileF32 A, B;
+    load_k(A, 0);
+    int64_t k = 0;
+    for (; k + 2 < ntot; k += 2) {
+      load_k(B, k + 1);
+      attend_k(A, k);
+      load_k(A, k + 2);
+      attend_k(B, k + 1);
+    }
+    if (k + 1 < ntot) {
+      load_k(B, k + 1);
+      attend_k(A, k);
+      attend_k(B, k + 1);
+    } else {
+      attend_k(A, k);
+    }
+  }
+
+  // ---- the output slice, or this split's partial slice for the merge launch
+  const bool direct = r.nact == 1 && a.gen_split < 0;
+  const int64_t base = (slot0 + sp) * T;
+  float l_tot = st.l_run + __shfl_xor(st.l_run, 16, kWave);
+  l_tot += __shfl_xor(l_tot, 32, kWave);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float li = __shfl(l_tot, 4 * g + i, kWave);
+    const int t = 4 * g + i;
+    if (t >= T) continue;
+    const float div = direct ? (li > 0.f ? li : 1.f) : 1.f;
+    float* dst = direct ? reinterpret_cast<float*>(a.out) + ((int64_t)(b * T + t) * a.H + h) * D
+                        : a.part_o + (base + t) * D;
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+      const int d = sl * 128 + 64 * nb + 4 * c;
+      const f32x4_t x = f32x4_t{o[4 * nb][i] / div, o[4 * nb + 1][i] / div, o[4 * nb + 2][i] / div,
+                                o[4 * nb + 3][i] / div};
+      if (direct || a.separate) *reinterpret_cast<f32x4_t*>(dst + d) = x;
+      else put_through4(a.part_o, (base + t) * D + d, x);
+    }
+  }
+  if (direct) return;
+  if (sl == 0 && g == 0 && c < T) {
+    if (a.separate) {
+      a.part_ml[(base + c) * 2] = st.m_ref;
+      a.part_ml[(base + c) * 2 + 1] = l_tot;
+    } else {
+      put_through2(a.part_ml + (base + c) * 2, st.m_ref, l_tot);
+    }
+  }
+  if (a.separate) return;
+  // The last split merges, as in verify_attn_slice_kernel.
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0);
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __syncthreads();
+  __shared__ int s_ticket;
+  int* counter = &a.counters[b * a.H + h];
+  if (threadIdx.x == 0) s_ticket = __hip_atomic_fetch_add(counter, 1, kTicketOrder, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (s_ticket != r.nact - 1) return;
+  merge_splits_fast<float>(a, b, h, r.nact, sl * 128, 128, slot0);
   if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -1463,16 +1681,23 @@ __global__ __launch_bounds__(64) void verify_attn_valu_kernel(AttnArgs a) {
 template <typename OutT, int DPL>
 __global__ __launch_bounds__(64) void verify_attn_combine_kernel(AttnArgs a) {
   const int t = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const SplitRange r = split_range(a, b, 0);
-  const int nact = r.nact;
+  int nact;
+  int64_t split0;
+  if (a.balanced) {  // the splits of the balanced deal (fp32)
+    const BalancedSplit bs = balanced_row(a, b);
+    nact = bs.nact;
+    split0 = (int64_t)h * a.splits + bs.first;
+  } else {
+    nact = split_range(a, b, 0).nact;
+    split0 = ((int64_t)b * a.H + h) * a.splits;
+  }
   if (nact == 1 && a.gen_split < 0) return;  // written directly by its only split
   const int nq = nact + (a.gen_split >= 0 ? 1 : 0);  // partials to merge
   const int lane = threadIdx.x;
   const int T = a.T, D = a.D;
-  const int64_t split0 = ((int64_t)b * a.H + h) * a.splits;
   OutT* orow = reinterpret_cast<OutT*>(a.out) + ((int64_t)(b * T + t) * a.H + h) * D;
   if (nq > kWave) {  // more partials than lanes to hold their (m, l): the generic merge
-    if (t == 0) merge_splits<OutT>(a, b, h, nact);
+    if (t == 0) merge_splits<OutT>(a, b, h, nact, split0);
     return;
   }
   const bool has_d = lane * DPL < D;
@@ -1583,6 +1808,12 @@ static int balanced_budget(int rows, int heads) {
   return per_head > rows ? per_head : rows;
 }
 
+// Waves of the fp32 launch in all, at most: one per SIMD.
+#ifndef OMNI_F32_WAVES
+#define OMNI_F32_WAVES 1024
+#endif
+constexpr int64_t kF32Waves = OMNI_F32_WAVES;
+
 static bool balanced_shape(int32_t rows, int32_t heads, int32_t head_dim) {
   // rows <= kBalancedMaxRows <= the workgroup's threads (one per row while the deal is computed)
   return (head_dim == 256 || head_dim == 512) && rows <= kBalancedMaxRows && balanced_budget(rows, heads) <= 65535;
@@ -1632,6 +1863,20 @@ extern "C" size_t omni_verify_attention_workspace(int32_t rows, int32_t tokens, 
   return align256(units * head_dim * sizeof(float)) + align256(units * 2 * sizeof(float));
 }
 
+// The fp32 MFMA kernel takes 16-byte rows at head dims 128, 256, 512; everything else in fp32 (and bf16 past the MFMA
+// shapes) stays on the vector ALU, whose loads are one element each.
+static bool f32_mfma(const AttnArgs& a, int dtype) {
+  return dtype == OMNI_F32 && (a.D == 128 || a.D == 256 || a.D == 512) && a.T <= 16 &&
+         (((uintptr_t)a.k | (uintptr_t)a.v) & 15u) == 0 && (a.s_row | a.s_head | a.s_pos) % 4 == 0 && a.s_pos >= 0 &&
+         a.s_pos < (1 << 24);  // 32-bit offsets within a tile
+}
+
+static void launch_f32(const AttnArgs& a, dim3 grid, hipStream_t s) {
+  if (a.D == 128) verify_attn_f32_kernel<128><<<grid, 64, 0, s>>>(a);
+  else if (a.D == 256) verify_attn_f32_kernel<256><<<grid, 128, 0, s>>>(a);
+  else verify_attn_f32_kernel<512><<<grid, 256, 0, s>>>(a);
+}
+
 // Key-split kernel and (when asked) the merge launch for filled-in arguments.
 static int launch_attention(const AttnArgs& a, int rows, int dtype, hipStream_t s) {
   const bool mfma = dtype == OMNI_BF16 && a.D % 128 == 0 && a.s_pos == a.D;  // contiguous key rows
@@ -1651,6 +1896,8 @@ static int launch_attention(const AttnArgs& a, int rows, int dtype, hipStream_t 
     }
   } else if (dtype == OMNI_BF16) {
     verify_attn_valu_kernel<uint16_t><<<grid, 64, 0, s>>>(a);
+  } else if (f32_mfma(a, dtype)) {
+    launch_f32(a, grid, s);
   } else {
     verify_attn_valu_kernel<float><<<grid, 64, 0, s>>>(a);
   }
@@ -1764,6 +2011,18 @@ extern "C" int omni_verify_attention(const void* q, const void* k_cache, const v
     // wide heads: a fixed budget of workgroups per head dealt to the rows by length, merged in the kernel
     launch_balanced_wide(a, rows, heads, head_dim, keys, s);
     return omni_launch_status();
+  }
+  if (a.separate && !(flags & OMNI_ATTN_SPLIT_K) && rows <= kBalancedMaxRows && f32_mfma(a, dtype)) {
+    // fp32: the same deal with a merge launch (no tickets, as split-K), one wave per SIMD in all where the workspace's
+    // slots allow it
+    const int64_t want = kF32Waves / (head_dim / 128) / heads, most = (int64_t)rows * attn_slots(keys, chunk);
+    a.balanced = 1;
+    a.splits = (int)(want < rows ? rows : want < most ? want : most);
+    a.ctx_splits = 1;
+    a.chunk = (keys + 31) / 32 * 32;
+    launch_f32(a, dim3(a.splits, heads, 1), s);
+    st = omni_launch_status();
+    return st != OMNI_OK ? st : launch_combine(a, rows, dtype, s);
   }
   st = launch_attention(a, rows, dtype, s);
   if (st != OMNI_OK || !a.separate) return st;

@@ -658,3 +658,26 @@ def test_spec_prepare_vs_oracle(cuda):
     for x, y in zip(got, want[:5]):
         np.testing.assert_array_equal(x.cpu().numpy().reshape(y.shape), y)
     np.testing.assert_array_equal(start.cpu().numpy(), want[5])
+
+
+@pytest.mark.parametrize("d,h,t,rows,separate", [
+    (128, 4, 1, 8, True), (128, 32, 16, 2, True), (256, 3, 5, 4, True), (512, 8, 5, 1, True), (512, 2, 16, 9, True),
+    (512, 1, 3, 70, True),  # more rows than the deal takes: plain key splits
+    (128, 2, 5, 5, False), (512, 2, 2, 6, False)])
+def test_verify_attention_f32_mfma(cuda, d, h, t, rows, separate):
+    """The fp32 MFMA kernel at the edges of its 16-key tiles (lengths 0, 1, 15, 16, 17, 31 .. and the whole cache), on
+    contiguous and on position-major caches ([rows, S, H, D] storage), with the merge launch and the in-kernel merge:
+    within the reference's fp32 tolerance (2e-5) of the fp64 oracle."""
+    g = gen(d + h + t + rows)
+    cap = 530
+    lengths = torch.tensor([0, 1, 15, 16, 17, 31, 300, 511, cap] * 8)[torch.randperm(72, generator=g)][:rows]
+    q = torch.randn(rows * t, h, d, generator=g)
+    kc, vc = torch.randn(rows, h, cap, d, generator=g), torch.randn(rows, h, cap, d, generator=g)
+    want = ov.verify_attention(npf(q), npf(kc), npf(vc), lengths.numpy(), t, d ** -0.5)
+    for major in (False, True):
+        say(f"fp32 attention d={d} h={h} t={t} rows={rows} separate={separate} position-major={major}")
+        kd, vd = ((x.transpose(1, 2).contiguous().to(cuda).transpose(1, 2) if major else x.to(cuda)) for x in (kc, vc))
+        out = kernels.draft_attention(q.to(cuda), kd, vd, lengths.to(cuda), t, 768, d ** -0.5, separate=separate)
+        torch.cuda.synchronize()
+        np.testing.assert_allclose(npf(out), want, atol=2e-5, rtol=2e-5)
+    assert int(kernels._counters[torch.cuda.current_device()].abs().sum()) == 0
