@@ -243,7 +243,7 @@ __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(2
   }
 }
 
-// Wide heads (D = 256, 512): one workgroup of kPwWaves waves per (query block, head, context).  The block's
+// Head dim 256: one workgroup of kPwWaves waves per (query block, head, context).  The block's
 // NG = kPwSub * M groups of 16 queries (M = kPwWaves / (D/128)): group gi holds queries qb + 16 gi .. + 15.  Wave w
 // holds the 128-dimension slice sl = w % (D/128) of q and O for the groups m + M u (m = w / (D/128), u < kPwSub).
 // Per 32-key tile (K and V through LDS once for all waves):
@@ -258,9 +258,9 @@ __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(2
 constexpr int kPwWaves = 8;
 constexpr int kPwSub = 3;  // 16-query groups per wave
 
-template <int D>
 __global__ __launch_bounds__(64 * kPwWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attn_wide_kernel(
     PrefillArgs a) {
+  constexpr int D = 256;
   constexpr int NSL = D / 128, M = kPwWaves / NSL, NG = kPwSub * M, QW = 16 * NG;
   constexpr int OWN = (NG + kPwWaves - 1) / kPwWaves;  // groups whose softmax one wave runs, at most
   constexpr int kRowB = D * 2 + 16;                     // LDS bytes per key row, padded against bank conflicts
@@ -486,6 +486,315 @@ __global__ __launch_bounds__(64 * kPwWaves) __attribute__((amdgpu_waves_per_eu(2
   }
 }
 
+// Head dim 512: one workgroup of 8 waves per 64 queries, two kinds of waves side by side on each SIMD.  Waves 0..3
+// ("scores") compute S^T = K Q^T, the softmax and P; waves 4..7 ("values") compute O^T += V^T P^T one 64-key tile
+// behind, so the softmax of a tile runs beside the matrix work of the one before, and a wave holds either Q (32 queries
+// x 512 dimensions, 128 registers) or O (64 queries x 128 dimensions, 128 registers), never both.  Both products are
+// v_mfma_f32_32x32x16_bf16.  One barrier per tile.
+//
+//  * Score wave w: queries 32 (w & 1) .. + 31, keys 32 (w >> 1) .. + 31 of the tile, all 512 dimensions.  Lane (x =
+//    lane % 32, g = lane / 32) gets query x's scores of keys 8 (i / 4) + 4g + i % 4, i < 16, and writes them as
+//    probabilities to LDS, 8 at a time: exactly the lane's B operand of O^T += V^T P^T.
+//  * Value wave w: dimensions 128w .. + 127 of all 64 queries.  V comes straight from memory into registers (each
+//    wave reads its own quarter of every row: nothing to share through LDS) in 16-byte loads, a whole tile ahead; a lane
+//    swap and a byte permute per operand dword transpose it.  Rows past the context read 0 (buffer bounds).  These
+//    waves also bring the next tile's K rows to LDS (global_load_lds, one 1 KB row each, rows 1040 bytes apart so
+//    that the 32 rows of an operand read start on different banks).
+//  * Softmax reference: a query's reference is the maximum of the first tile, and moves only when a score exceeds it
+//    by 2^kWsGuard (probabilities are relative, so fp32 and bf16 lose nothing; only their range is used).  Then, and
+//    on the first tile, the tile's two key halves exchange their maxima, P is written again and O is rescaled, between
+//    two more barriers (uniform over the workgroup: a flag every wave reads after the tile's barrier).
+//
+// What bounds a tile (64 queries x 64 keys): 2048 clocks of matrix work per SIMD, 2048 of the CU's vector memory path
+// (128 KB of K and V at 64 bytes a clock), 1860 of LDS; a tile takes ~3000, as a value wave issues its loads and its
+// products in one order.  The kernel this replaced added the partial scores of four 128-dimension slices through LDS,
+// with three barriers per 32 keys of 96 queries (5500 clocks for 1536 of matrix work).  Measured, 8 heads: 8 contexts
+// x 2048 521 -> 357 us (770 TFLOP/s); one context of 1433, where the longest block is the launch, 110 -> 39 us.  Tried:
+// 8-byte V loads of the operand's own rows, 390 / 45 us (the memory path takes a load instruction per 64 lanes, not
+// only its bytes); the loads spread between the products, 390-430 us (the tile's rows arrive later and its products
+// compete with the scores'); K rows brought by the score waves, 404 us; wave priorities, no change.
+constexpr int kWsD = 512, kWsQ = 64, kWsK = 64;
+constexpr int kWsRow = kWsD * 2 + 16;  // LDS bytes per K row
+constexpr int kWsAhead = 4;
+constexpr float kWsGuard = 16.0f;
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ f32x16_t mfma32(u32x4_t a, u32x4_t b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0,
+                                                 0, 0);
+}
+
+// A wave-uniform pointer in scalar registers.
+__device__ __forceinline__ const char* scalar_pointer(const void* p) {
+  const uint64_t u = reinterpret_cast<uint64_t>(p);
+  return reinterpret_cast<const char*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)u) |
+                                       (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32);
+}
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attn_ws_kernel(PrefillArgs a) {
+  constexpr int D = kWsD;
+  __shared__ __attribute__((aligned(16))) char kls[2][kWsK * kWsRow];
+  __shared__ u32x4_t ps[2][2][4][64];  // [tile parity][query half][16-key step][lane]
+  __shared__ float mxs[2][kWsQ];       // a tile's maxima by key half, when the reference moves
+  __shared__ float als[kWsQ];          // then: the factors O is rescaled by
+  __shared__ float lsum[2][2][kWsQ];   // at the end: probability sums by key half and lane half
+  __shared__ int moved[4];             // by tile % 4: a score passed the guard
+  const int nqb = (a.width + kWsQ - 1) / kWsQ;
+  const PfBlock blk = pf_block(nqb, a.H, (int)gridDim.z);
+  const int qb = (nqb - 1 - blk.j) * kWsQ;  // the longest blocks first
+  const int h = blk.h, b = blk.b;
+  const int tid = threadIdx.x, lane = tid & 63, x = lane & 31, g = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t slot = clamp64(a.slots[b], 0, a.cache_rows - 1);
+  const char* kbase = scalar_pointer(a.k + slot * a.s_row + h * a.s_head);
+  const char* vbase = scalar_pointer(a.v + slot * a.s_row + h * a.s_head);
+  const int nt = qb / kWsK + 1;  // the last tile holds the diagonal
+  if (tid < 4) moved[tid] = 0;
+
+  if (w < 4) {  // ------------------------------------------------------------------------------ scores
+    const int qh = w & 1, kh = w >> 1;
+    const int query = qb + 32 * qh + x;
+    u32x4_t q[D / 16];  // q[query][16s + 8g .. + 7] (past the end the last query's: its results are not stored)
+    {
+      const uint16_t* qrow = a.q + ((int64_t)(b * a.width + min(query, a.width - 1)) * a.H + h) * D + g * 8;
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) q[s] = *reinterpret_cast<const u32x4_t*>(qrow + s * 16);
+    }
+    float m_ref = -INFINITY, thr = -INFINITY, l_run = 0.f;
+    // K operands in a ring kWsAhead steps ahead of the products: an LDS read takes a few products' time to arrive.
+    u32x4_t kf[kWsAhead];
+    auto k_at = [&](int t, int s) {
+      return *reinterpret_cast<const u32x4_t*>(&kls[t & 1][(32 * kh + x) * kWsRow + g * 16 + s * 32]);
+    };
+    lds_barrier();  // the first K tile
+#pragma unroll
+    for (int s = 0; s < kWsAhead; ++s) kf[s] = k_at(0, s);
+    for (int t = 0; t < nt; ++t) {
+      f32x16_t s0, s1;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s0[i] = s1[i] = 0.f;
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) {
+        if (s & 1) s1 = mfma32(kf[s % kWsAhead], q[s], s1);
+        else s0 = mfma32(kf[s % kWsAhead], q[s], s0);
+        if (s + kWsAhead < D / 16) {
+          kf[s % kWsAhead] = k_at(t, s + kWsAhead);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one product, one LDS read
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+      }
+      float sv[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sv[i] = s0[i] + s1[i];
+      if (t == nt - 1) {
+        const int rel = query - (t * kWsK + 32 * kh + 4 * g);  // keys 8 (i / 4) + i % 4 <= rel are seen
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sv[i] = 8 * (i >> 2) + (i & 3) <= rel ? sv[i] : -INFINITY;
+      }
+      bool over = false;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) over |= sv[i] > thr;
+      if (__any(over) && lane == 0) moved[t & 3] = 1;
+      float lt = 0.f;
+      auto put_p = [&](float m) {
+        lt = 0.f;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          u32x4_t pop;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[8 * s + 2 * e], a.scale_log2, -m));
+            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[8 * s + 2 * e + 1], a.scale_log2, -m));
+            lt += p0 + p1;
+            pop[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{p0, p1}), bf16x2_t));
+          }
+          ps[t & 1][qh][2 * kh + s][lane] = pop;
+        }
+      };
+      put_p(m_ref == -INFINITY ? 0.f : m_ref);
+      lds_barrier();
+      const int again = moved[t & 3];  // uniform over the workgroup
+#pragma unroll
+      for (int s = 0; s < kWsAhead; ++s) kf[s] = k_at(t + 1, s);  // (past the last tile: unused)
+      if (w == 0 && lane == 0) moved[(t + 2) & 3] = 0;
+      if (again) {
+        float mx = sv[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, sv[i]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+        if (g == 0) mxs[kh][32 * qh + x] = mx;
+        lds_barrier();
+        const float m_new = fmaxf(m_ref, fmaxf(mxs[0][32 * qh + x], mxs[1][32 * qh + x]) * a.scale_log2);
+        const float alpha = __builtin_amdgcn_exp2f(m_ref - (m_new == -INFINITY ? 0.f : m_new));  // m_ref = -inf: 0
+        if (kh == 0 && g == 0) als[32 * qh + x] = alpha;
+        l_run *= alpha;
+        m_ref = m_new;
+        thr = m_new == -INFINITY ? -INFINITY : (m_new + kWsGuard) / a.scale_log2;
+        put_p(m_ref == -INFINITY ? 0.f : m_ref);
+        lds_barrier();
+      }
+      l_run += lt;
+    }
+    lsum[kh][g][32 * qh + x] = l_run;
+    lds_barrier();
+    return;
+  }
+
+  // ---------------------------------------------------------------------------------------------- values
+  const int vw = w - 4;
+  // [query half][e]: row r is dimension 128 vw + 8 (r % 16) + 4 (r / 16) + e, column x query x of the half
+  f32x16_t o[2][4];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[u][e][i] = 0.f;
+  // K rows 16 vw .. + 15 of tile t to LDS, one row (64 lanes x 16 bytes) per load; rows past the context read its last
+  // key (finite: masked).
+  const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kbase), 0, -1, 0x00020000);
+  auto bring_k = [&](int t) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int key = min(t * kWsK + 16 * vw + r, a.width - 1);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          kr, (__attribute__((address_space(3))) void*)&kls[t & 1][(16 * vw + r) * kWsRow], 16, lane * 16,
+          (int)((uint32_t)key * (D * 2)), 0,
+          0);
+    }
+  };
+  // V of 16-key step s of tile t: lane (c = x % 16, u = x / 16, g) loads keys 16s + 8u + 4g + j, dimensions 128 vw + 8c
+  // .. + 7, j < 4.  A buffer resource per step, its size what is left of the context's rows: scalar work only, and rows
+  // past the end read 0.
+  const uint32_t vlane = (uint32_t)((8 * (x >> 4) + 4 * g) * D + 128 * vw + 8 * (x & 15)) * 2;
+  const uint32_t vbytes = (uint32_t)a.width * (D * 2);
+  u32x4_t v[4][4];
+  auto load_v = [&](int t, int s) {
+    const uint32_t off = (uint32_t)(t * kWsK + 16 * s) * (D * 2);
+    uint32_t used = min(off, vbytes);
+    asm("" : "+s"(used));  // kept scalar (the saturating subtraction it would become is a vector instruction)
+    const __amdgpu_buffer_rsrc_t vr =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vbase) + off, 0, vbytes - used, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      v[s][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(vr, vlane + j * D * 2, 0, 0));
+  };
+  u32x4_t p[2][2];  // steps s, s + 1 of tile t
+  auto read_p = [&](int t, int s) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) p[u][s & 1] = ps[t & 1][u][s][lane];
+  };
+  // O^T += V^T P^T for tile t; ``ahead``: tile t + 1's V loads as its registers fall free.  Step s + 1's operands are
+  // built beside step s's products; the scheduler keeps each step's loads behind the permutes that read their registers.
+  auto attend_v = [&](int t, bool ahead) {
+    u32x4_t vop[2][4];
+    auto operands = [&](int s) {
+      // The lanes of a pair (u = 0, 1) hold 8 dimensions of 4 keys each; swapped, 4 dimensions (8c + 4u ..) of 8 keys:
+      // lo[j] of key 16s + 4g + j, hi[j] of key 16s + 8 + 4g + j.
+      u32x2_t lo[4], hi[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+          const auto r = __builtin_amdgcn_permlane16_swap(v[s][j][d], v[s][j][2 + d], false, false);
+          lo[j][d] = r[0];
+          hi[j][d] = r[1];
+        }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
+#pragma unroll
+        for (int q2 = 0; q2 < 2; ++q2) {
+          vop[s & 1][e][q2] = __builtin_amdgcn_perm(lo[2 * q2 + 1][e >> 1], lo[2 * q2][e >> 1], sel);
+          vop[s & 1][e][2 + q2] = __builtin_amdgcn_perm(hi[2 * q2 + 1][e >> 1], hi[2 * q2][e >> 1], sel);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(vop[s & 1][e]));  // built here, not where first used
+    };
+    operands(0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (ahead) load_v(t + 1, s);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) o[u][e] = mfma32(vop[s & 1][e], p[u][s & 1], o[u][e]);
+      if (s < 2) read_p(t, s + 2);
+      if (s < 3) operands(s + 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // After tile t's barrier: its probabilities, and O rescaled when the reference moved on it (O holds the tiles
+  // before it).
+  auto take_p = [&](int t) {
+    const int again = moved[t & 3];
+    read_p(t, 0);
+    read_p(t, 1);
+    if (!again) return;
+    lds_barrier();
+    lds_barrier();
+    read_p(t, 0);
+    read_p(t, 1);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const float al = als[32 * u + x];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[u][e][i] *= al;
+    }
+  };
+  bring_k(0);
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the tile is in LDS
+  lds_barrier();
+  bring_k(1);
+#pragma unroll
+  for (int s = 0; s < 4; ++s) load_v(0, s);
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  lds_barrier();
+  take_p(0);
+  for (int t = 1; t < nt; ++t) {  // tile t's scores, tile t - 1's values
+    bring_k(t + 1);  // unconditional (past the last tile: its last key's row, not used), so that no wait joins a branch
+    attend_v(t - 1, true);
+    // vmcnt(16): tile t + 1's K rows are in LDS, tile t's 16 V loads, issued after them, stay in flight (lds_barrier
+    // would wait for those too).  This wave's LDS reads of the tile are in registers by now.
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0x4f70);
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    take_p(t);
+  }
+  attend_v(nt - 1, false);
+  lds_barrier();
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int query = qb + 32 * u + x;
+    const float l = (lsum[0][0][32 * u + x] + lsum[0][1][32 * u + x]) + (lsum[1][0][32 * u + x] + lsum[1][1][32 * u + x]);
+    const float inv = l > 0.f ? 1.f / l : 1.f;
+    if (query >= a.width) continue;
+    uint16_t* orow = a.out + ((int64_t)(b * a.width + query) * a.H + h) * D + 128 * vw + 32 * g;
+    auto pair = [&](float lo, float hi) {
+      return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo * inv, hi * inv}), bf16x2_t));
+    };
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {  // dimensions 64r + 32g + 8i + 4k + e, k = 0, 1
+        u32x4_t out;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int at = 4 * (r + 2 * k) + i;
+          out[2 * k] = pair(o[u][0][at], o[u][1][at]);
+          out[2 * k + 1] = pair(o[u][2][at], o[u][3][at]);
+        }
+        *reinterpret_cast<u32x4_t*>(orow + 64 * r + 8 * i) = out;
+      }
+  }
+}
+
 }  // namespace omni
 
 extern "C" int omni_prefill_attention(const void* q, const void* k_cache, const void* v_cache, int64_t stride_row,
@@ -518,13 +827,13 @@ extern "C" int omni_prefill_attention(const void* q, const void* k_cache, const 
   if (head_dim == 128) {
     dim3 grid((width + omni::kPfQueries - 1) / omni::kPfQueries, heads, contexts);
     omni::prefill_attn_kernel<<<grid, 64 * omni::kPfWaves, 0, s>>>(a);
+  } else if (head_dim == 512) {
+    dim3 grid((width + omni::kWsQ - 1) / omni::kWsQ, heads, contexts);
+    omni::prefill_attn_ws_kernel<<<grid, 512, 0, s>>>(a);
   } else {
     const int qw = 16 * omni::kPwSub * (omni::kPwWaves / (head_dim / 128));  // queries per workgroup
     dim3 grid((width + qw - 1) / qw, heads, contexts);
-    if (head_dim == 256)
-      omni::prefill_attn_wide_kernel<256><<<grid, 64 * omni::kPwWaves, 0, s>>>(a);
-    else
-      omni::prefill_attn_wide_kernel<512><<<grid, 64 * omni::kPwWaves, 0, s>>>(a);
+    omni::prefill_attn_wide_kernel<<<grid, 64 * omni::kPwWaves, 0, s>>>(a);
   }
   return omni_launch_status();
 }

@@ -193,7 +193,7 @@ def test_verify_attention_wide_heads_up_to_32_queries(cuda, t, d):
 def test_prefill_attention(cuda, width, d, b, h):
     """Causal attention over whole contexts (src/omniasr_trt/decode.py:163-164) against the oracle's verify attention
     with query p of a context over keys [0, p]: cache rows addressed through slots, widths that are not multiples
-    of the query block (192 queries at head dims 128 and 256, 96 at 512) or of the 32-key tile; heads x contexts a
+    of the query block (192 queries at head dims 128 and 256, 64 at 512) or of the key tile; heads x contexts a
     multiple of 8 (the XCD-ordered workgroup map) or not (the plain one); at head dim 128 also widths past one
     block and up to six blocks."""
     g = gen(60 + width)
@@ -681,3 +681,28 @@ def test_verify_attention_f32_mfma(cuda, d, h, t, rows, separate):
         torch.cuda.synchronize()
         np.testing.assert_allclose(npf(out), want, atol=2e-5, rtol=2e-5)
     assert int(kernels._counters[torch.cuda.current_device()].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("width,b,h", [(1, 2, 3), (63, 1, 8), (64, 3, 8), (65, 1, 1), (129, 2, 4), (333, 1, 8)])
+@pytest.mark.parametrize("grow", [0.0, 40.0])
+def test_prefill_attention_512(cuda, width, b, h, grow):
+    """The head-dim 512 prefill at the edges of its 64-query blocks and 64-key tiles, one to six tiles.  ``grow``: scores
+    that climb along the context by far more than the softmax reference's guard, so that it moves on later tiles too.
+    Cache rows past the context hold NaN (stale memory): nothing of them may reach the output."""
+    g = gen(512 + width + b)
+    rows, cap, d = 4, -(-width // 64) * 64 + 32, 512
+    q = torch.randn(b * width, h, d, generator=g).to(torch.bfloat16)
+    kc = torch.randn(rows, h, cap, d, generator=g).to(torch.bfloat16)
+    vc = torch.randn(rows, h, cap, d, generator=g).to(torch.bfloat16)
+    if grow:  # the even dimensions of q positive, those of K rising with the position
+        q[..., ::2] = q[..., ::2].abs()
+        kc[..., ::2] = (kc[..., ::2] * 0.1 + grow * 0.1 * torch.arange(cap)[:, None] / width).to(torch.bfloat16)
+    slots = torch.tensor([3, 0, 2])[:b]
+    sl = slots.numpy()
+    want = ov.verify_attention(npf(q), npf(kc)[sl], npf(vc)[sl], np.ones(b, np.int64), width, d ** -0.5)
+    kc[:, :, width:] = float("nan")
+    vc[:, :, width:] = float("nan")
+    say(f"prefill attention 512 width={width} contexts={b} heads={h} grow={grow}")
+    out = kernels.prefill_attention(q.to(cuda), kc.to(cuda), vc.to(cuda), slots.to(cuda), width, d ** -0.5)
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(npf(out), want, atol=BF16_TOL[0], rtol=BF16_TOL[1])
