@@ -224,10 +224,9 @@ __device__ __forceinline__ f32x4_t get_through4(const float* base, int64_t at) {
 // The partials of (row b, head h) merged by one wave, each read at the coherence point: the row's ``nact`` key
 // splits from slot ``first_slot`` on (default: the unit's own slots), then the generated keys' partial if any (slot
 // ``gen_slot``; default: gen_split past the unit's first slot).
-template <typename OutT>
-__device__ void merge_splits_fast(const AttnArgs& a, int b, int h, int nact, int d0 = 0, int dw = -1,
-                                  int64_t first_slot = -1, int64_t gen_slot = -1) {
-  constexpr int kS = 8, kR = 3;
+template <typename OutT, int kS, int kR>
+__device__ __forceinline__ void merge_batches(const AttnArgs& a, int b, int h, int nact, int d0, int dw,
+                                              int64_t first_slot, int64_t gen_slot) {
   const int lane = lane_id();
   const int T = a.T, D = a.D;
   if (dw < 0) dw = D;  // dimensions d0 .. d0 + dw - 1 of every query (dw a multiple of 4)
@@ -293,6 +292,18 @@ __device__ void merge_splits_fast(const AttnArgs& a, int b, int h, int nact, int
       store4<OutT>(out + ((int64_t)(b * T + t) * a.H + h) * D + d0 + (f - t * dw), acc[r] / div);
     }
   }
+}
+
+// A batch is kS partials x kR x 256 floats, one memory round trip (~2 us at the coherence point) each: with few queries
+// a batch holds more partials, so the 32 splits of a lone row at 8 heads x 512 are one round trip instead of four
+// (one query over 1433 keys: 17.0 -> 13.1 us).
+template <typename OutT>
+__device__ void merge_splits_fast(const AttnArgs& a, int b, int h, int nact, int d0 = 0, int dw = -1,
+                                  int64_t first_slot = -1, int64_t gen_slot = -1) {
+  const int nf = a.T * (dw < 0 ? a.D : dw);
+  if (nact > 8 && nf <= 256) merge_batches<OutT, 32, 1>(a, b, h, nact, d0, dw, first_slot, gen_slot);
+  else if (nact > 8 && nf <= 512) merge_batches<OutT, 16, 2>(a, b, h, nact, d0, dw, first_slot, gen_slot);
+  else merge_batches<OutT, 8, 3>(a, b, h, nact, d0, dw, first_slot, gen_slot);
 }
 
 // After a split wrote its partial: the last of the row's ``nact`` splits merges them all.
@@ -464,7 +475,8 @@ __global__ __launch_bounds__(64, 2) void verify_attn_mfma_kernel(AttnArgs a) {
 // of tiles whatever the rows' lengths.  Workgroup j of a head works on split k of row b, one of the row's nact
 // splits (tiles dealt round-robin over them, as in split-K); the partials of a head's workgroups take the head's
 // a.splits slots in workgroup order, so a unit's splits have consecutive slots from ``first``.  Every workgroup
-// computes the same deal from the rows' lengths (rows <= kBalancedMaxRows).  b < 0: no work (every row empty).
+// computes the same deal from the rows' lengths (rows <= kBalancedMaxRows).  b < 0: no work (every row empty, or a
+// workgroup past the row's splits in use).
 // GEN: a row's tiles are its context tiles and then its beams' generated keys (see verify_attn_slice_kernel), whose
 // counts the deal leaves in gl[row][beam].
 constexpr int kBalancedMaxRows = 64;
@@ -479,6 +491,23 @@ __device__ __forceinline__ int gen_count(const AttnArgs& a, int64_t row) {
 struct BalancedSplit {
   int b, k, nact, first;
 };
+
+// Splits that work on a row of ``nt`` tiles dealt ``wk`` workgroups.  The row's last split reads every partial (T x D
+// floats each) through one CU, so a row alone on the chip is done sooner with fewer splits of more tiles: measured at 1
+// row x 8 heads x 512, a tile of a split costs ~1.5 us and a partial ~0.08 us per query (45 tiles, 5 queries: 32
+// splits 20.1 us, 23 18.1, 15 16.3, 12 16.7, 8 18.1; 9 queries over 16 tiles: 16 splits 19.0 us, 8 14.4; 16 queries
+// over 63 tiles: 32 41.1, 16 28.8, 8 27.6), so nt / n tiles and n T partials cost least at nt / n = sqrt(nt T / 18);
+// and no split is left with a tile less than the others (the same number of tiles each needs fewer of them).  Rows
+// that share the chip have 8 workgroups or fewer (one batch of the merge) and use them all.  Only the deal depends on
+// the result, within 1 .. wk, so approximate divisions do.
+__device__ __forceinline__ int splits_in_use(const AttnArgs& a, int nt, int wk) {
+  if (wk <= 8) return wk;
+  const float n = (float)nt;
+  float per = ceilf(n * __builtin_amdgcn_rcpf((float)wk) - 1e-3f);
+  if (!a.separate) per = fmaxf(per, rintf(__builtin_amdgcn_sqrtf(n * (float)a.T * (1.f / 18.f))));
+  const int use = (int)ceilf(n * __builtin_amdgcn_rcpf(fmaxf(per, 1.f)) - 1e-3f);
+  return use < 1 ? 1 : use > wk ? wk : use;
+}
 
 // Bit j: whether query c sees key 8g + j of a tile of a generated-key list (its keys' beam masks at msk8, in LDS).
 __device__ __forceinline__ int gen_bits(const uint16_t* msk8, int c) {
@@ -600,9 +629,9 @@ __global__ __launch_bounds__(256) void beam_gen_list_kernel(GenListArgs a) {
   if (tid == 0) a.count[grp] = total;
 }
 
-// The deal: wk[b] workgroups of each head for row b (LDS; the caller's rows <= blockDim.x).
+// The deal: wk[b] workgroups of each head for row b, the first na[b] of them at work (LDS; rows <= blockDim.x).
 template <bool GEN = false>
-__device__ __forceinline__ void balanced_deal(const AttnArgs& a, int* wk, int* gl = nullptr) {
+__device__ __forceinline__ void balanced_deal(const AttnArgs& a, int* wk, int* na, int* gl = nullptr) {
   __shared__ int nt[kBalancedMaxRows], rem[kBalancedMaxRows];
   __shared__ int s_total, s_given;
   const int tid = threadIdx.x, rows = a.rows, budget = a.splits;
@@ -620,6 +649,14 @@ __device__ __forceinline__ void balanced_deal(const AttnArgs& a, int* wk, int* g
     nt[tid] = n;
   }
   __syncthreads();
+  if (rows == 1) {
+    if (tid == 0) {
+      wk[0] = budget;
+      na[0] = splits_in_use(a, nt[0], budget);
+    }
+    __syncthreads();
+    return;
+  }
   if (tid == 0) {
     int total = 0;
     for (int b = 0; b < rows; ++b) total += nt[b];
@@ -628,9 +665,20 @@ __device__ __forceinline__ void balanced_deal(const AttnArgs& a, int* wk, int* g
   __syncthreads();
   const int total = s_total, spare = budget - rows;
   if (tid < rows) {
-    const int64_t share = total > 0 ? (int64_t)spare * nt[tid] : 0;
-    wk[tid] = 1 + (total > 0 ? (int)(share / total) : 0);
-    rem[tid] = total > 0 ? (int)(share % total) : 0;
+    uint32_t q = 0, m = 0;
+    if (total > 0) {
+      if ((uint64_t)spare * (uint32_t)total <= UINT32_MAX) {  // a 32-bit division is a fraction of a 64-bit one
+        const uint32_t share = (uint32_t)spare * (uint32_t)nt[tid];
+        q = share / (uint32_t)total;
+        m = share - q * (uint32_t)total;
+      } else {
+        const int64_t share = (int64_t)spare * nt[tid];
+        q = (uint32_t)(share / total);
+        m = (uint32_t)(share % total);
+      }
+    }
+    wk[tid] = 1 + (int)q;
+    rem[tid] = (int)m;
   }
   __syncthreads();
   if (tid == 0) {
@@ -647,20 +695,24 @@ __device__ __forceinline__ void balanced_deal(const AttnArgs& a, int* wk, int* g
     extra = rank < left;
   }
   __syncthreads();
-  if (tid < rows) wk[tid] += extra;
+  if (tid < rows) {
+    const int mine = wk[tid] + extra;
+    wk[tid] = mine;
+    na[tid] = splits_in_use(a, nt[tid], mine);
+  }
   __syncthreads();
 }
 
 // Workgroup j of a head: its row and split.
 template <bool GEN = false>
 __device__ BalancedSplit balanced_split(const AttnArgs& a, int j, int* gl = nullptr) {
-  __shared__ int wk[kBalancedMaxRows];
-  balanced_deal<GEN>(a, wk, gl);
+  __shared__ int wk[kBalancedMaxRows], na[kBalancedMaxRows];
+  balanced_deal<GEN>(a, wk, na, gl);
   BalancedSplit out{-1, 0, 1, 0};
   int first = 0;
   for (int b = 0; b < a.rows; ++b) {
     if (j < first + wk[b]) {
-      out = BalancedSplit{b, j - first, wk[b], first};
+      if (j < first + na[b]) out = BalancedSplit{b, j - first, na[b], first};
       break;
     }
     first += wk[b];
@@ -670,11 +722,11 @@ __device__ BalancedSplit balanced_split(const AttnArgs& a, int j, int* gl = null
 
 // Row b's splits of each head: their number and the first one's workgroup.
 __device__ __forceinline__ BalancedSplit balanced_row(const AttnArgs& a, int b) {
-  __shared__ int wk[kBalancedMaxRows];
-  balanced_deal<false>(a, wk);
+  __shared__ int wk[kBalancedMaxRows], na[kBalancedMaxRows];
+  balanced_deal<false>(a, wk, na);
   int first = 0;
   for (int o = 0; o < b; ++o) first += wk[o];
-  return BalancedSplit{b, 0, wk[b], first};
+  return BalancedSplit{b, 0, na[b], first};
 }
 
 // Split-K for head dims past 128 (256, 512): one workgroup of D/128 waves per (split, head, row), wave w holding

@@ -706,3 +706,17 @@ def test_prefill_attention_512(cuda, width, b, h, grow):
     out = kernels.prefill_attention(q.to(cuda), kc.to(cuda), vc.to(cuda), slots.to(cuda), width, d ** -0.5)
     torch.cuda.synchronize()
     np.testing.assert_allclose(npf(out), want, atol=BF16_TOL[0], rtol=BF16_TOL[1])
+
+
+@pytest.mark.parametrize("rows,h,t", [(1, 8, 1), (1, 8, 2), (1, 3, 5), (1, 8, 16), (2, 4, 3), (3, 8, 9), (1, 1, 5)])
+def test_verify_attention_wide_few_rows(cuda, rows, h, t):
+    """Few rows at head dim 512: rows dealt more than 8 workgroups put fewer of them to work and merge their partials in
+    batches of 32, 16 or 8.  From no keys over one tile to the whole cache, and 256 splits at one head (more than any
+    batch), against the oracle; the tickets are left zero."""
+    g = gen(7000 + rows + 10 * t)
+    cap, d = 2112, 512
+    for n in (0, 1, 32, 33, 500, 1433, cap):
+        lengths = torch.randint(0, cap + 1, (rows,), generator=g)
+        lengths[0] = n
+        _attn_case(cuda, torch.bfloat16, rows, h, d, t, cap, lengths, cap, 7100 + n, BF16_TOL)
+    assert int(kernels._counters[torch.cuda.current_device()].abs().sum()) == 0
