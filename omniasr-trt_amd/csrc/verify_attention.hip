@@ -1733,36 +1733,22 @@ __global__ __launch_bounds__(64) void verify_attn_valu_kernel(AttnArgs a) {
 template <typename OutT, int DPL>
 __global__ __launch_bounds__(64) void verify_attn_combine_kernel(AttnArgs a) {
   const int t = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  int nact;
-  int64_t split0;
-  if (a.balanced) {  // the splits of the balanced deal (fp32)
-    const BalancedSplit bs = balanced_row(a, b);
-    nact = bs.nact;
-    split0 = (int64_t)h * a.splits + bs.first;
-  } else {
-    nact = split_range(a, b, 0).nact;
-    split0 = ((int64_t)b * a.H + h) * a.splits;
-  }
-  if (nact == 1 && a.gen_split < 0) return;  // written directly by its only split
-  const int nq = nact + (a.gen_split >= 0 ? 1 : 0);  // partials to merge
   const int lane = threadIdx.x;
   const int T = a.T, D = a.D;
-  OutT* orow = reinterpret_cast<OutT*>(a.out) + ((int64_t)(b * T + t) * a.H + h) * D;
-  if (nq > kWave) {  // more partials than lanes to hold their (m, l): the generic merge
-    if (t == 0) merge_splits<OutT>(a, b, h, nact, split0);
-    return;
-  }
   const bool has_d = lane * DPL < D;
   const int d0 = has_d ? lane * DPL : 0;  // lanes past the head's dimensions read dimension 0 and store nothing
-  // The splits' rows in batches of kB, every load of a batch in flight at once (addresses clamped to the last
-  // split; the clamped repeats are not added), added in split order.  The first batch is issued before the
-  // splits' (m, l), which the weights need, so a merge of up to kB splits is one memory round trip.
+  // The partials' rows in batches of kB, every load of a batch in flight at once (slots clamped to the last one; the
+  // repeats are not added), added in split order, and the partials' (m, l), lane q holding partial q's.  Plain key
+  // splits take the slots from 0 on, so the first batch and the (m, l) load beside the row's length, which says how
+  // many of them count: one memory round trip for up to kB splits.
   constexpr int kB = 16;  // one batch for up to 16 splits (the default chunk gives at most 10 at 2560 keys)
   float po[kB][DPL];
-  auto load_batch = [&](int s0) {
+  float m, l;
+  int64_t split0 = ((int64_t)b * a.H + h) * a.splits;
+  auto load_batch = [&](int s0, int nact, int last) {
 #pragma unroll
     for (int j = 0; j < kB; ++j) {
-      const int sj = s0 + j < nq ? s0 + j : nq - 1;
+      const int sj = s0 + j < last ? s0 + j : last;
       const float* src = a.part_o + ((split0 + merge_slot(a, nact, sj)) * T + t) * D + d0;
       if constexpr (DPL % 4 == 0) {
 #pragma unroll
@@ -1777,13 +1763,37 @@ __global__ __launch_bounds__(64) void verify_attn_combine_kernel(AttnArgs a) {
       }
     }
   };
-  load_batch(0);
-  float m = -INFINITY, l = 0.f;
-  if (lane < nq) {
-    const int64_t ml = ((split0 + merge_slot(a, nact, lane)) * T + t) * 2;
+  auto load_ml = [&](int nact, int last) {
+    const int64_t ml = ((split0 + merge_slot(a, nact, lane < last ? lane : last)) * T + t) * 2;
     m = a.part_ml[ml];
     l = a.part_ml[ml + 1];
+  };
+  const bool early = !a.balanced && a.gen_split < 0;
+  if (early) {
+    load_batch(0, a.splits, a.splits - 1);
+    load_ml(a.splits, a.splits - 1);
   }
+  int nact;
+  if (a.balanced) {  // the splits of the balanced deal (fp32)
+    const BalancedSplit bs = balanced_row(a, b);
+    nact = bs.nact;
+    split0 = (int64_t)h * a.splits + bs.first;
+  } else {
+    nact = split_range(a, b, 0).nact;
+  }
+  if (nact == 1 && a.gen_split < 0) return;  // written directly by its only split
+  const int nq = nact + (a.gen_split >= 0 ? 1 : 0);  // partials to merge
+  OutT* orow = reinterpret_cast<OutT*>(a.out) + ((int64_t)(b * T + t) * a.H + h) * D;
+  if (nq > kWave) {  // more partials than lanes to hold their (m, l): the generic merge
+    if (t == 0) merge_splits<OutT>(a, b, h, nact, split0);
+    return;
+  }
+  if (!early) {
+    load_batch(0, nact, nq - 1);
+    load_ml(nact, nq - 1);
+  }
+  m = lane < nq ? m : -INFINITY;
+  l = lane < nq ? l : 0.f;
   const float top = wave_max(m);
   const float w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - top);
   const float den = wave_sum(w * l);
@@ -1801,7 +1811,7 @@ __global__ __launch_bounds__(64) void verify_attn_combine_kernel(AttnArgs a) {
       }
     }
     if (s0 + kB >= nq) break;
-    load_batch(s0 + kB);
+    load_batch(s0 + kB, nact, nq - 1);
   }
   if (!has_d) return;
 #pragma unroll
