@@ -66,22 +66,33 @@ __device__ __forceinline__ void load_tile_clamped(KVTile<D>& t, const char* kt, 
   }
 }
 
-// A tile of 32 gathered key rows into MFMA operand layout: ``rows`` (in LDS) holds the byte offset of each of the
-// tile's 32 keys from ``kt`` / ``vt`` (the same offset in K and V); every offset is a key in use.
-template <int D>
-__device__ __forceinline__ void load_tile_rows(KVTile<D>& t, const char* kt, const char* vt, const uint32_t* rows, int c,
-                                               int g) {
+// A tile of a unit whose tiles are context keys and then gathered ones, into MFMA operand layout.  ``gathered`` (wave-
+// uniform): the tile's 32 key rows are at the byte offsets ``rows`` (LDS, each a key in use) from ``kt`` / ``vt``, the
+// same in K and V; otherwise the tile is load_tile_clamped's (``rows`` is read all the same, any 32 entries).  Only
+// addresses are selected, so one set of loads serves both kinds: with the two kinds' loads under a branch the wait at
+// its join covers every load in flight, and the next tile's loads no longer overlap this tile's math (measured, the
+// beams' attention of 12 layers at 8 inputs x 5 beams, 64 generated keys: 704 -> 680 us at 8 heads x 512, 686 -> 669 at
+// 32 x 128; 2 inputs, 3 generated keys: 265 -> 254 us).
+template <int D, uint32_t kRow = D * 2>
+__device__ __forceinline__ void load_tile_either(KVTile<D>& t, const char* kt, const char* vt, bool gathered,
+                                                 const uint32_t* rows, int kmax, int vstop, int c, int g) {
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb) {
-    const uint32_t ko = rows[8 * (c >> 2) + 4 * mb + (c & 3)] + g * 16;
+    const int r = 8 * (c >> 2) + 4 * mb + (c & 3);
+    const uint32_t at = rows[r], row = (uint32_t)(r < kmax ? r : kmax) * kRow;
+    const uint32_t ko = (gathered ? at : row) + g * 16;
 #pragma unroll
     for (int s = 0; s < KVTile<D>::KS; ++s) t.k[mb][s] = ld16(kt + ko + s * 64);
   }
+  int vmax = vstop - 1 < kmax ? vstop - 1 : kmax;
+  vmax = vmax > 0 ? vmax : 0;
   const u32x4_t r0 = *reinterpret_cast<const u32x4_t*>(rows + 8 * g);
   const u32x4_t r1 = *reinterpret_cast<const u32x4_t*>(rows + 8 * g + 4);
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const uint32_t vo = (j < 4 ? r0[j] : r1[j - 4]) + c * 16;
+    const int rv = 8 * g + j;
+    const uint32_t at = j < 4 ? r0[j] : r1[j - 4], row = (uint32_t)(rv < vmax ? rv : vmax) * kRow;
+    const uint32_t vo = (gathered ? at : row) + c * 16;
 #pragma unroll
     for (int gg = 0; gg < KVTile<D>::NG; ++gg) t.v[gg][j] = ld16(vt + vo + gg * 256);
   }

@@ -488,6 +488,25 @@ __device__ __forceinline__ int gen_count(const AttnArgs& a, int64_t row) {
   return (int)clamp64(a.gen_len[row], 0, a.gen_cap);
 }
 
+// The generated keys in use, into LDS, every load in one round trip (the caller's barrier follows): with the step's list
+// only each group's count, gl[group T]; otherwise every beam's, gl[row].  A group's thread reads its own list count back
+// (gen_keys) without a barrier.
+__device__ __forceinline__ void load_gen_counts(const AttnArgs& a, int groups, int* gl, int nt) {
+  if (a.glist) {
+    for (int g = threadIdx.x; g < groups; g += nt) gl[g * a.T] = min(a.gcount[g], a.gen_table);  // at most the table
+  } else {
+    for (int i = threadIdx.x; i < groups * a.T; i += nt) gl[i] = gen_count(a, i);
+  }
+}
+
+// Group b's generated keys (a list's length, or its beams' keys).
+__device__ __forceinline__ int gen_keys(const AttnArgs& a, int b, const int* gl) {
+  int n = gl[b * a.T];
+  if (!a.glist)
+    for (int e = 1; e < a.T; ++e) n += gl[b * a.T + e];
+  return n;
+}
+
 struct BalancedSplit {
   int b, k, nact, first;
 };
@@ -635,17 +654,13 @@ __device__ __forceinline__ void balanced_deal(const AttnArgs& a, int* wk, int* n
   __shared__ int nt[kBalancedMaxRows], rem[kBalancedMaxRows];
   __shared__ int s_total, s_given;
   const int tid = threadIdx.x, rows = a.rows, budget = a.splits;
+  if constexpr (GEN) {
+    load_gen_counts(a, rows, gl, blockDim.x);
+    if (!a.glist) __syncthreads();
+  }
   if (tid < rows) {
     int n = (int)((split_range(a, tid, 0).total + 31) >> 5);
-    if constexpr (GEN) {
-      int ng = 0;
-      for (int e = 0; e < a.T; ++e) {
-        const int ne = gen_count(a, (int64_t)tid * a.T + e);
-        gl[tid * a.T + e] = ne;
-        ng += ne;
-      }
-      n += ((a.glist ? min(a.gcount[tid], a.gen_table) : ng) + 31) >> 5;
-    }
+    if constexpr (GEN) n += (gen_keys(a, tid, gl) + 31) >> 5;
     nt[tid] = n;
   }
   __syncthreads();
@@ -799,9 +814,7 @@ __global__ __launch_bounds__(64 * (D / 128), G == 1 ? 2 : 1) void verify_attn_sl
   const char* kgb = nullptr;
   const char* vgb = nullptr;
   if constexpr (GEN) {
-    int ng = 0;
-    for (int e = 0; e < T; ++e) ng += s_gl[b * T + e];
-    ng = __builtin_amdgcn_readfirstlane(a.glist ? min(a.gcount[b], a.gen_table) : ng);  // a list holds at most the table
+    const int ng = __builtin_amdgcn_readfirstlane(gen_keys(a, b, s_gl));
     row_tiles += (ng + 31) >> 5;
     kgb = a.kg + h * a.g_head * 2 + sl * 256;
     vgb = a.vg + h * a.g_head * 2 + sl * 256;
@@ -818,10 +831,13 @@ __global__ __launch_bounds__(64 * (D / 128), G == 1 ? 2 : 1) void verify_attn_sl
   auto load_k = [&](KVTile<128>& t, int64_t k) {
     if constexpr (GEN) {
       const int ti = (int)(first + k * r.nact);
-      if (ti >= ctx_tiles) {  // a tile of generated keys (wave-uniform)
-        load_tile_rows<128>(t, kgb, vgb, s_tab + (ti - ctx_tiles) * 32, c, g);
-        return;
-      }
+      const bool gt = ti >= ctx_tiles;  // a tile of generated keys (wave-uniform)
+      const int64_t kb = (int64_t)(gt ? 0 : ti) * 32;
+      const int64_t kmax = last_key - kb, vstop = r.total - kb;
+      load_tile_either<128, D * 2>(t, gt ? kgb : kt + k * tile_bytes, gt ? vgb : vt + k * tile_bytes, gt,
+                                   s_tab + (gt ? ti - ctx_tiles : 0) * 32, kmax < 31 ? (int)kmax : 31,
+                                   vstop < 32 ? (int)vstop : 32, c, g);
+      return;
     }
     const int64_t kb = (first + k * r.nact) * 32;
     const int64_t kmax = last_key - kb, vstop = r.total - kb;
@@ -852,11 +868,16 @@ __global__ __launch_bounds__(64 * (D / 128), G == 1 ? 2 : 1) void verify_attn_sl
         }
       }
       const int ti = (int)(first + k * r.nact);
-      if (GEN && ti >= ctx_tiles)  // generated keys: the beams that see each key
-        attend_scored<128, true>(t, tot, a.scale_log2, st[u], o[u], g, 0,
-                                 u == 0 ? gen_bits(s_msk + (ti - ctx_tiles) * 32 + 8 * g, c) : 0);
-      else
+      if constexpr (GEN) {  // each lane's mask, from the keys' beams or the context's length (one code path for both)
+        const bool gt = ti >= ctx_tiles;
+        const int gb = gen_bits(s_msk + (gt ? ti - ctx_tiles : 0) * 32 + 8 * g, c);
+        int cb = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) cb |= ti * 32 + 8 * g + j < lim_c[u] ? 1 << j : 0;
+        attend_scored<128, true>(t, tot, a.scale_log2, st[u], o[u], g, 0, gt ? gb : cb);
+      } else {
         attend_scored<128>(t, tot, a.scale_log2, st[u], o[u], g, ti * 32 + 8 * g, lim_c[u]);
+      }
     }
   };
   // The buffer written for tile k was last read for tile k - 2, before every wave passed tile k - 1's barrier.
@@ -1299,17 +1320,13 @@ __global__ __launch_bounds__(64 * kWgWaves, 1) void verify_attn_pair_kernel(Attn
   uint32_t* tab = reinterpret_cast<uint32_t*>(s_gl + ((rows * T + 3) & ~3));  // 16-byte aligned (row reads)
   uint16_t* msk = reinterpret_cast<uint16_t*>(tab + 2 * a.gen_table);
   if (tid == 0) s_done = 0;
+  if constexpr (GEN) {
+    load_gen_counts(a, rows, s_gl, 64 * kWgWaves);
+    if (!a.glist) __syncthreads();
+  }
   for (int b = tid; b < rows; b += 64 * kWgWaves) {
     int nt = row_tile_count(a, b);
-    if constexpr (GEN) {
-      int ng = 0;
-      for (int e = 0; e < T; ++e) {
-        const int n = gen_count(a, (int64_t)b * T + e);
-        s_gl[b * T + e] = n;
-        ng += n;
-      }
-      nt += ((a.glist ? min(a.gcount[b], a.gen_table) : ng) + 31) >> 5;
-    }
+    if constexpr (GEN) nt += (gen_keys(a, b, s_gl) + 31) >> 5;
     ntl[b] = nt;
   }
   __syncthreads();
@@ -1327,11 +1344,7 @@ __global__ __launch_bounds__(64 * kWgWaves, 1) void verify_attn_pair_kernel(Attn
   const SplitRange r0 = split_range(a, b0, 0), r1 = split_range(a, b1, 0);
   const int nc0 = (int)((r0.total + 31) >> 5), nc1 = (int)((r1.total + 31) >> 5);  // context tiles
   // GEN: the units' generated keys (wave-uniform)
-  auto gen_total = [&](int bu) {
-    int n = 0;
-    for (int e = 0; e < T; ++e) n += s_gl[bu * T + e];
-    return __builtin_amdgcn_readfirstlane(a.glist ? min(a.gcount[bu], a.gen_table) : n);  // at most the table
-  };
+  auto gen_total = [&](int bu) { return __builtin_amdgcn_readfirstlane(gen_keys(a, bu, s_gl)); };
   const int ng0 = GEN ? gen_total(b0) : 0, ng1 = GEN ? gen_total(b1) : 0;
   const int nt0 = nc0 + ((ng0 + 31) >> 5), nt1 = nc1 + ((ng1 + 31) >> 5);
   const int e0 = (nt0 + 1) >> 1, s1 = (nt1 + 1) >> 1;  // half 0: tiles [0, e0) of u0; half 1: [s1, nt1) of u1
@@ -1409,11 +1422,17 @@ __global__ __launch_bounds__(64 * kWgWaves, 1) void verify_attn_pair_kernel(Attn
     const int tile = tile_of(k);
     if constexpr (GEN) {
       const int nc = first ? nc0 : nc1;
-      if (tile >= nc) {  // a tile of generated keys (wave-uniform)
-        load_tile_rows<D>(t, first ? kgb0 : kgb1, first ? vgb0 : vgb1,
-                          tab + (first ? 0 : a.gen_table) + (tile - nc) * 32, c, g);
-        return;
-      }
+      const bool gt = tile >= nc;  // a tile of generated keys (wave-uniform)
+      const int64_t k0 = (int64_t)(gt ? 0 : tile) * 32, off = k0 * D * 2;
+      const int64_t kmax = last_key - k0, vstop = (first ? r0.total : r1.total) - k0;
+      const char* kc = first ? kb0 : kb1;
+      const char* vc = first ? vb0 : vb1;
+      const char* kg = first ? kgb0 : kgb1;
+      const char* vg = first ? vgb0 : vgb1;
+      load_tile_either<D>(t, gt ? kg : kc + off, gt ? vg : vc + off, gt,
+                          tab + (first ? 0 : a.gen_table) + (gt ? tile - nc : 0) * 32, kmax < 31 ? (int)kmax : 31,
+                          vstop < 32 ? (int)vstop : 32, c, g);
+      return;
     }
     ld_tile(t, first ? kb0 : kb1, first ? vb0 : vb1, tile, first ? r0.total : r1.total);
   };
