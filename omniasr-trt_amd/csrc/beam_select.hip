@@ -13,8 +13,11 @@
 //
 // Layout: one 256-thread workgroup per row (the log-softmax needs the whole row; a row is ~20 KB, so one workgroup
 // per row spreads the group's reads over N CUs): the row's max and sum are two workgroup reductions in a fixed order;
-// each offer and its flat index become one 64-bit key ordered as the choice is, so each wave takes its N best in N
-// rounds of a branch-free scan and a wave-wide maximum, and wave 0 merges the waves' lists into the row's N best.
+// each offer's value becomes a 32-bit number ordered as the choice is.  The N-th largest of a wave's threads' bests is a
+// floor under the row's N best, so only the offers at or above the largest floor (few more than N) become 64-bit keys,
+// value above inverted index, and wave 0 ranks them by counting.  What bounds it is that chain at one row's size, not
+// the 20 KB: as N rounds of a 64-bit scan of all offers and a wave-wide maximum, at three levels, the launch took 18 us (now 11)
+// at 8 groups x 5 beams x 10288; those rounds remain for rows with more than 256 offers at the floor (equal values).
 // The row writes them through to the device's coherence point (the rows of a group run on different XCDs, whose L2s
 // are not coherent) and takes the group's ticket; the last row of the group reads the N rows' lists and merges them
 // into the group's N best.  Every selection is by (value, index), so the result does not depend on which row
@@ -29,15 +32,18 @@ namespace omni {
 constexpr int kSelThreads = 256;
 constexpr int kSelWaves = kSelThreads / kWave;
 constexpr int kSelMaxBeams = 16;
+constexpr int kSelCand = 256;  // candidates of a row in LDS (and the N x N keys of a group, at most 256)
 
 // An offer and its flat index as one 64-bit key whose unsigned order is the choice's order: the value's bits mapped
 // to an order-preserving unsigned integer (negative values bit-inverted, positive ones with the sign bit set; -0 as
 // +0, so equal values stay equal) above the index inverted (a lower index is the larger key).  Keys are unique, and 0
-// is below every offer's key.
-__device__ __forceinline__ uint64_t sel_key(float v, int i) {
-  uint32_t b = v == 0.f ? 0u : __float_as_uint(v);
-  const uint32_t u = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-  return ((uint64_t)u << 32) | (uint64_t)(0xffffffffu - (uint32_t)i);
+// is below every offer's key, in its value half as in the whole.
+__device__ __forceinline__ uint32_t sel_order(float v) {
+  const uint32_t b = v == 0.f ? 0u : __float_as_uint(v);
+  return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+}
+__device__ __forceinline__ uint64_t sel_key(uint32_t order, int i) {
+  return ((uint64_t)order << 32) | (uint64_t)(0xffffffffu - (uint32_t)i);
 }
 __device__ __forceinline__ float sel_value(uint64_t k) {
   const uint32_t u = (uint32_t)(k >> 32);
@@ -55,19 +61,33 @@ __device__ __forceinline__ uint64_t sel_wave_max(uint64_t k) {
   return k;
 }
 
-// The wave's n largest of its lanes' E keys each, in order: lane j < n gets the j-th (0 past the keys there are).
-template <int E>
-__device__ __forceinline__ uint64_t sel_wave_top(const uint64_t (&keys)[E], int n) {
-  uint64_t prev = ~0ull, mine = 0;
-  for (int j = 0; j < n; ++j) {
-    uint64_t best = 0;
-#pragma unroll
-    for (int e = 0; e < E; ++e) best = keys[e] < prev && keys[e] > best ? keys[e] : best;
-    best = sel_wave_max(best);
-    if (lane_id() == j) mine = best;
-    prev = best;
+// The wave's largest 32-bit value, on the data-parallel lane moves (a cross-lane read through LDS takes ~10 times as
+// long): within rows of 16 lanes, then across them; lanes without a source take 0.
+template <int kCtrl>
+__device__ __forceinline__ uint32_t sel_dpp_max(uint32_t v) {
+  const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xf, 0xf, false);
+  return o > v ? o : v;
+}
+__device__ __forceinline__ uint32_t sel_wave_max32(uint32_t v) {
+  v = sel_dpp_max<0x111>(v);  // row_shr 1, 2, 4, 8: lane 15 of each row holds the row's
+  v = sel_dpp_max<0x112>(v);
+  v = sel_dpp_max<0x114>(v);
+  v = sel_dpp_max<0x118>(v);
+  v = sel_dpp_max<0x142>(v);  // row_bcast 15, 31: lane 63 holds the wave's
+  v = sel_dpp_max<0x143>(v);
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// keys[0 .. m) in LDS, unique: lanes' own keys (lane, lane + 64, ...) by rank; ``put(rank, key)`` for the n best.
+template <typename Put>
+__device__ __forceinline__ void sel_rank(const uint64_t* keys, int m, int n, Put put) {
+  for (int i = lane_id(); i < m; i += kWave) {
+    const uint64_t mine = keys[i];
+    int rank = 0;
+#pragma unroll 4
+    for (int j = 0; j < m; ++j) rank += keys[j] > mine;
+    if (rank < n) put(rank, mine);
   }
-  return mine;
 }
 
 __device__ __forceinline__ float sel_block_reduce(float v, float* red, bool is_max) {
@@ -106,7 +126,9 @@ template <int CPT>
 __global__ __launch_bounds__(kSelThreads) void beam_select_kernel(SelectArgs a) {
 #pragma clang fp contract(off)
   __shared__ float red[kSelWaves];
-  __shared__ uint64_t wk[kSelWaves][kSelMaxBeams];
+  __shared__ uint64_t cand[kSelCand];
+  __shared__ uint32_t wave_floor[kSelWaves];
+  __shared__ int n_cand;
   const int row = blockIdx.x, n = a.beams, V = a.vocab;
   const int g = row / n, b = row - g * n;
   const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
@@ -143,9 +165,10 @@ __global__ __launch_bounds__(kSelThreads) void beam_select_kernel(SelectArgs a) 
     logsum = logf(sum);
   }
 
-  // The row's offers as keys with their flat indices in the group's N x V (past V: key 0, never chosen).
-  uint64_t keys[CPT * 8];
+  // The row's offers' orders (past V: 0, never chosen).
+  uint32_t ord[CPT * 8];
   const float cf = (float)cnt, c1 = (float)(cnt + 1);
+  uint32_t cur = 0;  // this thread's best
 #pragma unroll
   for (int c = 0; c < CPT; ++c)
 #pragma unroll
@@ -159,25 +182,73 @@ __global__ __launch_bounds__(kSelThreads) void beam_select_kernel(SelectArgs a) 
       } else {
         o = score + lp;
       }
-      if (ended) o = v == a.eos ? score : -INFINITY;
-      keys[c * 8 + e] = v < V ? sel_key(o, b * V + v) : 0ull;
+      const uint32_t order = sel_order(o);
+      ord[c * 8 + e] = v < V ? (order > 1u ? order : 1u) : 0u;
+      cur = ord[c * 8 + e] > cur ? ord[c * 8 + e] : cur;
     }
 
-  // Each wave's N best, then wave 0 merges the waves' lists into the row's.
-  const uint64_t mine = sel_wave_top<CPT * 8>(keys, n);
-  if (lane < n) wk[wave][lane] = mine;
-  __syncthreads();
-  if (wave != 0) return;
-  uint64_t mk[1];
-  {
-    const int w = lane / kSelMaxBeams, j = lane - w * kSelMaxBeams;  // kSelWaves x kSelMaxBeams = 64 lanes
-    mk[0] = j < n ? wk[w][j] : 0ull;
+  // The row's candidates, in LDS.  A finished row offers EOS at its score and -inf elsewhere: its N best are among EOS
+  // and the first N + 1 tokens.  Otherwise n threads of a wave hold an offer of at least the n-th largest of the
+  // threads' bests, so the row's N best are at or above the largest of the waves' N-th: few more than N unless values
+  // tie.
+  if (tid == 0) n_cand = 0;
+  if (!ended) {  // block-uniform
+    uint32_t floor_w = 0;
+    for (int j = 0; j < n; ++j) {
+      floor_w = sel_wave_max32(cur);
+      const uint64_t at = __ballot(cur == floor_w);
+      if (lane == __ffsll((unsigned long long)at) - 1) cur = 0;
+    }
+    if (lane == 0) wave_floor[wave] = floor_w;
   }
-  const uint64_t rowk = sel_wave_top<1>(mk, n);
+  __syncthreads();
+  if (ended) {
+    const int few = n + 1 < V ? n + 1 : V;
+    if (tid < few) cand[tid] = sel_key(sel_order(tid == a.eos ? score : -INFINITY), b * V + tid);
+    if (tid == 0) {
+      const bool extra = a.eos >= few && a.eos < V;
+      if (extra) cand[few] = sel_key(sel_order(score), b * V + (int)a.eos);
+      n_cand = few + (extra ? 1 : 0);
+    }
+  } else {
+    uint32_t least = wave_floor[0];
+#pragma unroll
+    for (int w = 1; w < kSelWaves; ++w) least = wave_floor[w] > least ? wave_floor[w] : least;
+    least = least > 1u ? least : 1u;
+#pragma unroll
+    for (int i = 0; i < CPT * 8; ++i)
+      if (ord[i] >= least) {
+        const int at = __hip_atomic_fetch_add(&n_cand, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (at < kSelCand) cand[at] = sel_key(ord[i], b * V + (tid + (i >> 3) * kSelThreads) * 8 + (i & 7));
+      }
+  }
+  __syncthreads();
+  const int found = n_cand;  // block-uniform
+  if (found > kSelCand) {  // many equal values: each wave's N best in N rounds, in the candidates' place
+    __syncthreads();
+    uint64_t prev = ~0ull, mine = 0;
+    for (int j = 0; j < n; ++j) {
+      uint64_t best = 0;
+#pragma unroll
+      for (int i = 0; i < CPT * 8; ++i) {
+        const uint64_t k = ord[i] ? sel_key(ord[i], b * V + (tid + (i >> 3) * kSelThreads) * 8 + (i & 7)) : 0ull;
+        best = k < prev && k > best ? k : best;
+      }
+      best = sel_wave_max(best);
+      if (lane == j) mine = best;
+      prev = best;
+    }
+    if (lane < n) cand[wave * n + lane] = mine;
+    __syncthreads();
+  }
+  if (wave != 0) return;
+  const int have = found > kSelCand ? kSelWaves * n : found;
 
   // The row's list, written through; then the group's ticket.
   uint64_t* crow = a.cand + (int64_t)row * n;
-  if (lane < n) __hip_atomic_store(crow + lane, rowk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  sel_rank(cand, have, n, [&](int rank, uint64_t k) {
+    __hip_atomic_store(crow + rank, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  });
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __builtin_amdgcn_s_waitcnt(0);
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -192,15 +263,17 @@ __global__ __launch_bounds__(kSelThreads) void beam_select_kernel(SelectArgs a) 
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int f = lane + q * kWave;
-    const bool have = f < n * n;
-    const uint64_t k = __hip_atomic_load(cg + (have ? f : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    gk[q] = have ? k : 0ull;
+    gk[q] = __hip_atomic_load(cg + (f < n * n ? f : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  const uint64_t gkey = sel_wave_top<4>(gk, n);
-  if (lane < n) {
-    a.best[(int64_t)g * n + lane] = sel_value(gkey);
-    a.flat[(int64_t)g * n + lane] = sel_index(gkey);
-  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (lane + q * kWave < n * n) cand[lane + q * kWave] = gk[q];
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");  // this wave's own reads follow
+  __builtin_amdgcn_s_waitcnt(0xc07f);                              // lgkmcnt(0): the keys are in LDS
+  sel_rank(cand, n * n, n, [&](int rank, uint64_t k) {
+    a.best[(int64_t)g * n + rank] = sel_value(k);
+    a.flat[(int64_t)g * n + rank] = sel_index(k);
+  });
   if (lane == 0) __hip_atomic_store(a.tickets + g, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 

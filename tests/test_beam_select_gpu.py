@@ -166,3 +166,35 @@ def test_beam_select_refusals(cuda):
     assert not kernels.beam_select_supported(torch.zeros(10, 16392, dtype=torch.bfloat16, device=cuda), sc, 5)
     with pytest.raises(ValueError):
         kernels.beam_select(lg, sc, ct, en, 3, False, EOS)  # 10 rows: not groups of 3
+
+
+@pytest.mark.parametrize("beams,vocab", [(1, 64), (5, 64), (16, 512), (5, 10288), (16, 16384), (3, 2048)])
+@pytest.mark.parametrize("values", ["spread", "few", "one"])
+def test_beam_select_ties_and_finished_rows(cuda, beams, vocab, values):
+    """The choice by (value, lower flat index) on log-probabilities of few distinct values -- so many offers tie at the
+    floor that they do not fit the candidates (one value: all of them) -- and of many; with finished rows whose EOS is
+    among the first tokens or far behind them, and whose frozen score is finite or -inf: indices and values equal a
+    stable sort of the offers torch's own ops make."""
+    groups, g = 4, torch.Generator().manual_seed(beams * vocab)
+    rows = groups * beams
+    scale = {"spread": 4.0, "few": 0.02, "one": 0.0}[values]
+    logits = (torch.randn(rows, vocab, generator=g) * scale).to(torch.bfloat16).to(cuda)
+    score = -torch.rand(rows, generator=g) * 3
+    ended = torch.rand(rows, generator=g) < 0.3
+    score[ended.nonzero()[:1]] = float("-inf")
+    count = torch.randint(1, 9, (rows,), generator=g)
+    score, ended, count = score.to(cuda), ended.to(cuda), count.to(cuda)
+    for eos in (2, vocab - 1):
+        for norm in (False, True):
+            logp = torch.nn.functional.log_softmax(logits, dim=-1)
+            s, c = score[:, None], count[:, None]
+            offers = (s * c + logp) / (c + 1) if norm else s + logp
+            offers = offers.masked_fill(ended[:, None], float("-inf"))
+            offers[:, eos] = torch.where(ended, score, offers[:, eos])
+            flat = offers.view(groups, -1).cpu()
+            want = torch.sort(flat, dim=-1, descending=True, stable=True)
+            print(f"beam_select ties beams={beams} vocab={vocab} {values} eos={eos} norm={norm}", flush=True)
+            best, idx = kernels.beam_select(logits, score, count, ended, beams, norm, eos)
+            torch.cuda.synchronize()
+            assert torch.equal(best.cpu(), want.values[:, :beams])
+            assert torch.equal(idx.cpu(), want.indices[:, :beams])
