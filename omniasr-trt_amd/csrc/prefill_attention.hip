@@ -9,23 +9,11 @@
 
 namespace omni {
 
-// Causal attention over whole contexts (the prefill): query p of context b attends to keys [0, p] of its cache row.
-// One workgroup of kPfWaves waves per (query block, head, context), the longest blocks first.  The block's 32-key
-// tiles go through LDS once for all of its waves (double-buffered: tile t + 1's global loads are in flight during
-// tile t's math).  Each wave holds kPfSub groups of 16 queries: per tile it reads the K fragments and, by LDS
-// transpose reads, the V operands once, then runs S^T = K Q^T, the lazy softmax (causal limit as the key limit,
-// skipped on tiles the whole group sees) and O += P V for every group that sees the tile.
-constexpr int kPfWaves = 4;
-constexpr int kPfSub = 3;  // 16-query groups per wave (3: 255 VGPRs, two waves per SIMD; measured fastest of 1-4)
-constexpr int kPfQueries = 16 * kPfSub * kPfWaves;
-constexpr int kPfRow = 128 * 2 + 16;  // LDS bytes per key row: 256 B of data, padded against bank conflicts
-constexpr int kPfStage = 32;          // keys per LDS stage (one barrier each), a multiple of the 32-key MFMA tile
-constexpr int kPfThreads = 64 * kPfWaves;
+// Query p of context b attends to keys [0, p] of its cache row; one workgroup per (query block, head, context), the
+// longest blocks first; every kernel keeps a lazy softmax reference and masks only the tiles on the diagonal.
 typedef short v4i16_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4i16_t lds_v4i16;
 typedef __attribute__((address_space(3))) const char lds_char;
-constexpr int kPfChunks = kPfStage * 16 / kPfThreads;  // 16-byte chunks of K (and of V) per thread per stage
-static_assert(kPfChunks * kPfThreads == kPfStage * 16, "a stage is whole chunks per thread");
 
 struct PrefillArgs {
   const uint16_t* q;    // [B * width, H, D] bf16
@@ -52,195 +40,6 @@ __device__ __forceinline__ PfBlock pf_block(int nqb, int H, int B) {
   const int x = L % 8, k = L / 8;
   const int unit = (k / nqb) * 8 + x;
   return PfBlock{k % nqb, unit % H, unit / H};
-}
-
-// The softmax step of one 16-query group for one tile: mask (key0 + j >= lim), lazy reference max, this lane's
-// 8 probabilities packed as the P operand.  (The same arithmetic as attend().)
-template <int NB>
-__device__ __forceinline__ u32x4_t softmax_tile(float (&sv)[8], float c_scale, SoftmaxState& st, f32x4_t (&o)[NB],
-                                                int g, int key0, int lim, bool whole) {
-  bool over = false;
-  if (!whole) {  // whole (wave-uniform): every query of the group sees every key of the tile
-#pragma unroll
-    for (int j = 0; j < 8; ++j) sv[j] = key0 + j < lim ? sv[j] : -INFINITY;
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) over |= sv[j] > st.thr;
-  if (__any(over)) {
-    float mx = sv[0];
-#pragma unroll
-    for (int j = 1; j < 8; ++j) mx = fmaxf(mx, sv[j]);
-    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-    const float m_new = fmaxf(st.m_ref, mx * c_scale);
-    rescale<NB>(st.m_ref, m_new == -INFINITY ? 0.f : m_new, st.l_run, o, g);
-    st.m_ref = m_new;
-    st.thr = m_new == -INFINITY ? -INFINITY : (m_new + kLazyLog2) / c_scale;
-  }
-  const float m_use = st.m_ref == -INFINITY ? 0.f : st.m_ref;
-  float p[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    p[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[j], c_scale, -m_use));
-    st.l_run += p[j];
-  }
-  u32x4_t pop;
-#pragma unroll
-  for (int w = 0; w < 4; ++w)
-    pop[w] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{p[2 * w], p[2 * w + 1]}), bf16x2_t));
-  return pop;
-}
-
-__global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attn_kernel(
-    PrefillArgs a) {
-  constexpr int D = 128, KS = D / 32;
-  __shared__ __attribute__((aligned(16))) char lds[2][2][kPfStage * kPfRow];  // [buffer][K, V][key rows]
-  const int nqb = (a.width + kPfQueries - 1) / kPfQueries;
-  const PfBlock blk = pf_block(nqb, a.H, (int)gridDim.z);
-  const int qb = (nqb - 1 - blk.j) * kPfQueries;  // the longest blocks first
-  const int h = blk.h, b = blk.b;
-  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t slot = clamp64(a.slots[b], 0, a.cache_rows - 1);
-  const uint16_t* kbase = a.k + slot * a.s_row + h * a.s_head;
-  const uint16_t* vbase = a.v + slot * a.s_row + h * a.s_head;
-  const int kend = min(qb + kPfQueries, a.width);  // keys the block's last query sees
-  const int nt = (kend + kPfStage - 1) / kPfStage;
-
-  // Global -> LDS: thread tid moves 16-byte chunks tid, tid + kPfThreads, ... of the stage's K and of its V (kPfStage rows x
-  // 256 B each).  Rows past the context read its last key (finite: masked by the causal limit, never NaN).
-  u32x4_t stage[2 * kPfChunks];
-  auto fetch = [&](int t) {
-#pragma unroll
-    for (int e = 0; e < kPfChunks; ++e) {
-      const int ci = tid + e * kPfThreads, r = ci >> 4, col = ci & 15;
-      const int key = min(t * kPfStage + r, a.width - 1);
-      stage[e] = *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)key * D + col * 8);
-      stage[kPfChunks + e] = *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)key * D + col * 8);
-    }
-  };
-  auto put = [&](int buf) {
-#pragma unroll
-    for (int e = 0; e < kPfChunks; ++e) {
-      const int ci = tid + e * kPfThreads, r = ci >> 4, col = ci & 15;
-      *reinterpret_cast<u32x4_t*>(&lds[buf][0][r * kPfRow + col * 16]) = stage[e];
-      *reinterpret_cast<u32x4_t*>(&lds[buf][1][r * kPfRow + col * 16]) = stage[kPfChunks + e];
-    }
-  };
-
-  // The wave's groups: queries q0[u] + c, u < kPfSub (group u of wave w: block rows 16 (w + kPfWaves u)).
-  int q0[kPfSub];
-  u32x4_t qop[kPfSub][KS];  // B operand of S^T = K Q^T: lane (c, g) holds q[q0 + c][32s + 8g .. +7] (0 past the end)
-  SoftmaxState st[kPfSub];
-  f32x4_t o[kPfSub][D / 16];
-#pragma unroll
-  for (int u = 0; u < kPfSub; ++u) {
-    q0[u] = qb + 16 * (w + kPfWaves * u);
-    const bool live = q0[u] + c < a.width;
-    const uint16_t* qrow = a.q + ((int64_t)(b * a.width + (live ? q0[u] + c : 0)) * a.H + h) * D + g * 8;
-#pragma unroll
-    for (int s2 = 0; s2 < KS; ++s2)
-      qop[u][s2] = live ? *reinterpret_cast<const u32x4_t*>(qrow + s2 * 32) : u32x4_t{0u, 0u, 0u, 0u};
-    st[u] = SoftmaxState{-INFINITY, -INFINITY, 0.f};
-#pragma unroll
-    for (int nb = 0; nb < D / 16; ++nb) o[u][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
-
-  fetch(0);
-  put(0);
-  __syncthreads();
-  for (int t = 0; t < nt; ++t) {
-    fetch(t + 1 < nt ? t + 1 : t);  // unconditional: the last iteration re-reads its own tile (cache hit)
-    // The stage's 32-key MFMA tiles in turn.
-#pragma unroll
-    for (int sub = 0; sub < kPfStage / 32; ++sub) {
-    const int key0 = t * kPfStage + sub * 32;
-    // Groups that see the tile (wave-uniform): a live group whose last query reaches the tile's first key.
-    bool act[kPfSub];
-    bool any = false;
-#pragma unroll
-    for (int u = 0; u < kPfSub; ++u) {
-      act[u] = q0[u] < a.width && key0 <= q0[u] + 15;
-      any |= act[u];
-    }
-    if (any) {
-      const char* kl = lds[t & 1][0] + sub * 32 * kPfRow;
-      const char* vl = lds[t & 1][1] + sub * 32 * kPfRow;
-      u32x4_t pop[kPfSub];
-      {
-        u32x4_t kf[2][KS];
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb) {
-          const int rk = 8 * (c >> 2) + 4 * mb + (c & 3);
-#pragma unroll
-          for (int s2 = 0; s2 < KS; ++s2) kf[mb][s2] = *reinterpret_cast<const u32x4_t*>(kl + rk * kPfRow + g * 16 + s2 * 64);
-        }
-#pragma unroll
-        for (int u = 0; u < kPfSub; ++u) {
-          if (!act[u]) continue;
-          f32x4_t sacc[2];
-#pragma unroll
-          for (int mb = 0; mb < 2; ++mb) {
-            sacc[mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int s2 = 0; s2 < KS; ++s2)
-              sacc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[mb][s2]),
-                                                                 __builtin_bit_cast(bf16x8_t, qop[u][s2]), sacc[mb],
-                                                                 0, 0, 0);
-          }
-          float sv[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) sv[j] = sacc[j >> 2][j & 3];
-          pop[u] = softmax_tile<D / 16>(sv, a.scale_log2, st[u], o[u], g, key0 + 8 * g, q0[u] + c + 1,
-                                        key0 + 31 <= q0[u]);
-        }
-      }
-      {
-        // V operands by transpose reads: in lane group g (keys 8g .. 8g + 7) lane 4r + q points at key
-        // 8g + 4h + r, dimensions 16e + 4q .. 16e + 4q + 3 (h = 0, 1), and ds_read_b64_tr_b16 hands lane c the
-        // four keys' dimension 16e + c: block e's B operand, output column c = dimension 16e + c.
-        const int rr = c >> 2, q4 = c & 3;
-        const lds_char* vls = (const lds_char*)vl;  // vl points into LDS
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int off = (8 * g + rr) * kPfRow + (16 * e + 4 * q4) * 2;
-          const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vls + off));
-          const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vls + off + 4 * kPfRow));
-          u32x4_t bop;
-          bop[0] = (uint32_t)(uint16_t)lo[0] | ((uint32_t)(uint16_t)lo[1] << 16);
-          bop[1] = (uint32_t)(uint16_t)lo[2] | ((uint32_t)(uint16_t)lo[3] << 16);
-          bop[2] = (uint32_t)(uint16_t)hi[0] | ((uint32_t)(uint16_t)hi[1] << 16);
-          bop[3] = (uint32_t)(uint16_t)hi[2] | ((uint32_t)(uint16_t)hi[3] << 16);
-#pragma unroll
-          for (int u = 0; u < kPfSub; ++u) {
-            if (!act[u]) continue;
-            o[u][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, pop[u]),
-                                                              __builtin_bit_cast(bf16x8_t, bop), o[u][e], 0, 0, 0);
-          }
-        }
-      }
-    }
-    }
-    put((t + 1) & 1);
-    __syncthreads();
-  }
-
-  // ---- each group's 16 output rows: O / l, rounded to bf16
-#pragma unroll
-  for (int u = 0; u < kPfSub; ++u) {
-    float l_tot = st[u].l_run + __shfl_xor(st[u].l_run, 16, kWave);
-    l_tot += __shfl_xor(l_tot, 32, kWave);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float li = __shfl(l_tot, 4 * g + i, kWave);
-      const int qq = q0[u] + 4 * g + i;
-      if (qq >= a.width) continue;
-      const float div = li > 0.f ? li : 1.f;
-      uint16_t* orow = a.out + ((int64_t)(b * a.width + qq) * a.H + h) * D;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) orow[16 * e + c] = (uint16_t)pack_bf16x2(o[u][e][i] / div, 0.f);  // dim 16e + c
-    }
-  }
 }
 
 // Head dim 256: one workgroup of kPwWaves waves per (query block, head, context).  The block's
@@ -795,6 +594,272 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
+// Head dim 128: 256 queries per workgroup, four pairs of a score wave and a value wave (see prefill_attn_ws_kernel), each
+// pair its own 64 queries against the same 64-key tiles.  Score wave p of step t multiplies tile t (K from LDS, Q in
+// registers) beside the softmax of tile t - 1, so its matrix and vector work overlap within the wave; value wave p
+// accumulates tile t - 2.  A pair keeps its own softmax reference (a lane's two queries see every key of the tile
+// through lanes x and x + 32), so a moved reference costs no barrier: the factors wait in LDS for the value wave.
+// K and V rows go to LDS by direct loads (score waves bring V, value waves K: neither reads what it brings, so no wait
+// for the loads comes before the barrier), 1 KB = 4 rows each, 16-byte chunks permuted within a row so that the
+// operand reads spread over the banks: chunk c of key r at position c ^ (r % 16) in K, c ^ 4 (r % 4) in V.
+//
+// What bounds a tile (a pair's 64 queries x 64 keys): 2048 clocks of matrix work on its SIMD beside ~1900 of the score
+// wave's vector work (64 exponentials per lane at a quarter rate), one barrier per tile.  The kernel this replaced ran
+// both in one wave, one after the other, on 16 x 16 products with 192 queries per workgroup.  Measured, 32 heads, before
+// and after: 4 contexts x 1777 203 -> 147 us (705 TFLOP/s), 8 x 2048 405 -> 362 us (760), one of 1433 64 -> 42 us, 8 of
+// 130 16 -> 13 us.  Tried: fmaxf in place of max3, 157 / 387 us; K operands 3 steps ahead (3 registers spilled) with
+// the products and the vector work interleaved by sched_group_barrier, 151 / 378 us; wave priorities, no change.
+constexpr int kPairQ = 256, kPairK = 64;
+
+// Without the copy of each operand that fmaxf makes to quiet a signalling NaN (a product has none).  The compiler does
+// not see an instruction that reads a, b, c here: a caller with values of the matrix unit waits for them first.
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attn_pairs_kernel(
+    PrefillArgs a) {
+  constexpr int D = 128;
+  __shared__ __attribute__((aligned(16))) char kls[2][kPairK * D * 2];
+  __shared__ __attribute__((aligned(16))) char vls[2][kPairK * D * 2];
+  __shared__ u32x4_t ps[4][2][2][4][64];  // [pair][tile parity][query half][16-key step][lane]
+  __shared__ float als[4][4][64];         // [pair][tile % 4]: O's factors, when the reference moved
+  __shared__ int moved[4][4];
+  __shared__ float lsum[4][2][64];        // [pair][lane half]
+  const int nqb = (a.width + kPairQ - 1) / kPairQ;
+  const PfBlock blk = pf_block(nqb, a.H, (int)gridDim.z);
+  const int qb = (nqb - 1 - blk.j) * kPairQ;  // the longest blocks first
+  const int h = blk.h, b = blk.b;
+  const int tid = threadIdx.x, lane = tid & 63, x = lane & 31, g = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), pr = w & 3;
+  const int64_t slot = clamp64(a.slots[b], 0, a.cache_rows - 1);
+  const char* kbase = scalar_pointer(a.k + slot * a.s_row + h * a.s_head);
+  const char* vbase = scalar_pointer(a.v + slot * a.s_row + h * a.s_head);
+  const int nt = (min(qb + kPairQ, a.width) + kPairK - 1) / kPairK;
+  const int qp = qb + 64 * pr;
+  const int dq = qp < a.width ? qp / kPairK : -1;  // the pair's last tile, which holds its diagonal (-1: no queries)
+
+  // Rows 16 pr .. + 15 of tile t to LDS; rows past the context read its last key (finite: masked).  ``swap``: the chunk
+  // permutation of key row r of a 16-row group.
+  auto bring = [&](const __amdgpu_buffer_rsrc_t rsrc, char* dst, int t, auto swap) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = 4 * j + (lane >> 4);
+      const int key = min(t * kPairK + 16 * pr + r, a.width - 1);
+      const uint32_t from = (uint32_t)key * (D * 2) + (uint32_t)((lane & 15) ^ swap(r)) * 16;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rsrc, (__attribute__((address_space(3))) void*)(dst + (16 * pr + 4 * j) * (D * 2)), 16, from, 0, 0, 0);
+    }
+  };
+
+  if (w < 4) {  // ------------------------------------------------------------------------------ scores
+    const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vbase), 0, -1, 0x00020000);
+    auto bring_v = [&](int t) { bring(vr, vls[t & 1], t, [](int r) { return 4 * (r & 3); }); };
+    u32x4_t q[2][D / 16];  // q[query][16s + 8g .. + 7], query qp + 32u + x
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const uint16_t* qrow =
+          a.q + ((int64_t)(b * a.width + min(qp + 32 * u + x, a.width - 1)) * a.H + h) * D + g * 8;
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) q[u][s] = *reinterpret_cast<const u32x4_t*>(qrow + s * 16);
+    }
+    float m_ref[2] = {-INFINITY, -INFINITY}, thr[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
+    const int klane = x * (D * 2) + ((g ^ (x & 15)) * 16);
+    auto k_at = [&](int t, int m, int s) {
+      return *reinterpret_cast<const u32x4_t*>(&kls[t & 1][32 * m * (D * 2) + (klane ^ (32 * s))]);
+    };
+    typedef f32x16_t Scores[2][2];  // [key half m][query half u]
+    f32x16_t zero;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) zero[i] = 0.f;
+    // One 16-key step's probabilities of query half u: keys 16 (2m + hf) .., as the value wave's operand.
+    auto put_p = [&](const Scores& sc, int t, int m, int hf, int u, float mu) {
+      u32x4_t pop;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[m][u][8 * hf + 2 * e], a.scale_log2, -mu));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[m][u][8 * hf + 2 * e + 1], a.scale_log2, -mu));
+        l_run[u] += p0 + p1;
+        pop[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{p0, p1}), bf16x2_t));
+      }
+      ps[pr][t & 1][u][2 * m + hf][lane] = pop;
+    };
+    // The reference of tile t's scores (masked on the pair's last tile).
+    auto refer = [&](Scores& sc, int t) {
+      // max3's operands come from the matrix unit: every product has written its result after 24 wait states.
+      asm volatile("s_nop 15\n\ts_nop 7" : "+v"(sc[0][0]), "+v"(sc[0][1]), "+v"(sc[1][0]), "+v"(sc[1][1]));
+      if (t == dq) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int rel = 32 * u + x - (32 * m + 4 * g);  // keys 8 (i / 4) + i % 4 <= rel are seen
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sc[m][u][i] = 8 * (i >> 2) + (i & 3) <= rel ? sc[m][u][i] : -INFINITY;
+          }
+      }
+      float mx[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        mx[u] = max3(sc[0][u][0], sc[1][u][0], sc[0][u][1]);
+        mx[u] = max3(mx[u], sc[1][u][1], sc[1][u][1]);
+#pragma unroll
+        for (int i = 2; i < 16; ++i) mx[u] = max3(mx[u], sc[0][u][i], sc[1][u][i]);
+      }
+      const bool move = __any(mx[0] > thr[0] || mx[1] > thr[1]);
+      if (lane == 0) moved[pr][t & 3] = move ? 1 : 0;
+      if (move) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const float top = fmaxf(mx[u], __shfl_xor(mx[u], 32, kWave));
+          const float m_new = fmaxf(m_ref[u], top * a.scale_log2);
+          const float alpha = __builtin_amdgcn_exp2f(m_ref[u] - (m_new == -INFINITY ? 0.f : m_new));  // m_ref = -inf: 0
+          if (g == 0) als[pr][t & 3][32 * u + x] = alpha;
+          l_run[u] *= alpha;
+          m_ref[u] = m_new;
+          thr[u] = m_new == -INFINITY ? -INFINITY : (m_new + kWsGuard) / a.scale_log2;
+        }
+      }
+    };
+    // Step t: tile t's products into ``to``, the softmax of tile t - 1's scores ``from`` beside them.
+    auto step = [&](const Scores& from, Scores& to, int t, bool soft) {
+      u32x4_t kf[2] = {k_at(t, 0, 0), k_at(t, 1, 0)};
+      const float m0 = m_ref[0] == -INFINITY ? 0.f : m_ref[0], m1 = m_ref[1] == -INFINITY ? 0.f : m_ref[1];
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) to[m][u] = mfma32(kf[m], q[u][s], s == 0 ? zero : to[m][u]);
+        if (s + 1 < D / 16) {
+#pragma unroll
+          for (int m = 0; m < 2; ++m) kf[m] = k_at(t, m, s + 1);
+        }
+        if (soft) put_p(from, t - 1, s >> 2, (s >> 1) & 1, s & 1, s & 1 ? m1 : m0);
+      }
+      refer(to, t);
+    };
+    auto finish = [&](const Scores& from, int t) {  // the pair's last tile
+      const float m0 = m_ref[0] == -INFINITY ? 0.f : m_ref[0], m1 = m_ref[1] == -INFINITY ? 0.f : m_ref[1];
+#pragma unroll
+      for (int s = 0; s < 8; ++s) put_p(from, t, s >> 2, (s >> 1) & 1, s & 1, s & 1 ? m1 : m0);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) lsum[pr][g][32 * u + x] = l_run[u];
+    };
+    Scores sa, sb;
+    lds_barrier();  // the first K tile
+    if (dq >= 0) step(sb, sa, 0, false);
+    lds_barrier();
+    int t = 1;
+    for (; t + 1 <= dq; t += 2) {
+      bring_v(t - 1);
+      step(sa, sb, t, true);
+      lds_barrier();
+      bring_v(t);
+      step(sb, sa, t + 1, true);
+      lds_barrier();
+    }
+    if (t <= dq) {  // one more, then its scores are in sb
+      bring_v(t - 1);
+      step(sa, sb, t, true);
+      lds_barrier();
+      bring_v(t);
+      finish(sb, t);
+      lds_barrier();
+      t += 2;
+    } else if (dq >= 0) {
+      bring_v(t - 1);
+      finish(sa, t - 1);
+      lds_barrier();
+      t += 1;
+    }
+    for (; t <= nt + 1; ++t) {
+      if (t <= nt) bring_v(t - 1);
+      lds_barrier();
+    }
+    return;
+  }
+
+  // ---------------------------------------------------------------------------------------------- values
+  const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kbase), 0, -1, 0x00020000);
+  auto bring_k = [&](int t) { bring(kr, kls[t & 1], t, [](int r) { return r; }); };
+  f32x16_t o[2][4];  // [query half][e]: row 16k + 4q + i is dimension 32e + 8q + 4k + i, column x query x of the half
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[u][e][i] = 0.f;
+  // V operands by transpose reads: within 16 lanes (k = lane / 16 % 2), lane 4r + q points at key 4g + r, dimensions
+  // 32e + 8q + 4k .., and lane 4q + i receives dimension 32e + 8q + 4k + i of the four keys.
+  const int r = (lane & 15) >> 2, q4 = lane & 3, k2 = (lane >> 4) & 1;
+  int vlane[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) vlane[e] = (4 * g + r) * (D * 2) + (e ^ r) * 64 + q4 * 16 + k2 * 8;
+  auto attend_v = [&](int t) {
+    u32x4_t p[2][4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) p[u][s] = ps[pr][t & 1][u][s][lane];
+    if (moved[pr][t & 3]) {  // wave-uniform
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const float al = als[pr][t & 3][32 * u + x];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[u][e][i] *= al;
+      }
+    }
+    const lds_char* vt = (const lds_char*)vls[t & 1];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vt + vlane[e] + s * 16 * D * 2));
+        const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vt + vlane[e] + (s * 16 + 8) * D * 2));
+        const u32x2_t l2 = __builtin_bit_cast(u32x2_t, lo), h2 = __builtin_bit_cast(u32x2_t, hi);
+        const u32x4_t vop = {l2[0], l2[1], h2[0], h2[1]};
+#pragma unroll
+        for (int u = 0; u < 2; ++u) o[u][e] = mfma32(vop, p[u][s], o[u][e]);
+      }
+  };
+  bring_k(0);
+  lds_barrier();
+  for (int t = 0; t <= nt + 1; ++t) {
+    if (t + 1 < nt) bring_k(t + 1);
+    if (t >= 2 && t - 2 <= dq) attend_v(t - 2);
+    lds_barrier();
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int query = qp + 32 * u + x;
+    if (query >= a.width) continue;
+    const float l = lsum[pr][0][32 * u + x] + lsum[pr][1][32 * u + x];
+    const float inv = l > 0.f ? 1.f / l : 1.f;
+    uint16_t* orow = a.out + ((int64_t)(b * a.width + query) * a.H + h) * D + 8 * g;
+    auto pair = [&](float lo, float hi) {
+      return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo * inv, hi * inv}), bf16x2_t));
+    };
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {  // dimensions 32e + 16 rb + 8g .. + 7
+        u32x4_t out;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int at = 4 * (rb + 2 * k);
+          out[2 * k] = pair(o[u][e][at], o[u][e][at + 1]);
+          out[2 * k + 1] = pair(o[u][e][at + 2], o[u][e][at + 3]);
+        }
+        *reinterpret_cast<u32x4_t*>(orow + 32 * e + 16 * rb) = out;
+      }
+  }
+}
+
 }  // namespace omni
 
 extern "C" int omni_prefill_attention(const void* q, const void* k_cache, const void* v_cache, int64_t stride_row,
@@ -825,13 +890,13 @@ extern "C" int omni_prefill_attention(const void* q, const void* k_cache, const 
   a.out = (uint16_t*)out;
   hipStream_t s = (hipStream_t)stream;
   if (head_dim == 128) {
-    dim3 grid((width + omni::kPfQueries - 1) / omni::kPfQueries, heads, contexts);
-    omni::prefill_attn_kernel<<<grid, 64 * omni::kPfWaves, 0, s>>>(a);
+    dim3 grid((width + omni::kPairQ - 1) / omni::kPairQ, heads, contexts);
+    omni::prefill_attn_pairs_kernel<<<grid, 512, 0, s>>>(a);
   } else if (head_dim == 512) {
     dim3 grid((width + omni::kWsQ - 1) / omni::kWsQ, heads, contexts);
     omni::prefill_attn_ws_kernel<<<grid, 512, 0, s>>>(a);
   } else {
-    const int qw = 16 * omni::kPwSub * (omni::kPwWaves / (head_dim / 128));  // queries per workgroup
+    const int qw = 16 * omni::kPwSub * (omni::kPwWaves / 2);  // queries per workgroup
     dim3 grid((width + qw - 1) / qw, heads, contexts);
     omni::prefill_attn_wide_kernel<<<grid, 64 * omni::kPwWaves, 0, s>>>(a);
   }

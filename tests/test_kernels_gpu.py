@@ -193,9 +193,9 @@ def test_verify_attention_wide_heads_up_to_32_queries(cuda, t, d):
 def test_prefill_attention(cuda, width, d, b, h):
     """Causal attention over whole contexts (src/omniasr_trt/decode.py:163-164) against the oracle's verify attention
     with query p of a context over keys [0, p]: cache rows addressed through slots, widths that are not multiples
-    of the query block (192 queries at head dims 128 and 256, 64 at 512) or of the key tile; heads x contexts a
+    of the query block (256 queries at head dim 128, 192 at 256, 64 at 512) or of the key tile; heads x contexts a
     multiple of 8 (the XCD-ordered workgroup map) or not (the plain one); at head dim 128 also widths past one
-    block and up to six blocks."""
+    block and up to five blocks."""
     g = gen(60 + width)
     rows, cap = 5, max(448, -(-width // 64) * 64)
     kc = torch.randn(rows, h, cap, d, generator=g).to(torch.bfloat16)
@@ -720,3 +720,28 @@ def test_verify_attention_wide_few_rows(cuda, rows, h, t):
         lengths[0] = n
         _attn_case(cuda, torch.bfloat16, rows, h, d, t, cap, lengths, cap, 7100 + n, BF16_TOL)
     assert int(kernels._counters[torch.cuda.current_device()].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("width,b,h", [(1, 2, 3), (63, 1, 8), (64, 3, 8), (65, 1, 1), (255, 1, 8), (257, 2, 4),
+                                       (450, 1, 8), (641, 1, 2)])
+@pytest.mark.parametrize("grow", [0.0, 40.0])
+def test_prefill_attention_128(cuda, width, b, h, grow):
+    """The head-dim 128 prefill at the edges of its 64-query pairs, 256-query blocks and 64-key tiles: blocks with one to
+    four live pairs, odd and even numbers of tiles.  ``grow`` and the stale rows as in test_prefill_attention_512."""
+    g = gen(128 + width + b)
+    rows, cap, d = 4, -(-width // 64) * 64 + 32, 128
+    q = torch.randn(b * width, h, d, generator=g).to(torch.bfloat16)
+    kc = torch.randn(rows, h, cap, d, generator=g).to(torch.bfloat16)
+    vc = torch.randn(rows, h, cap, d, generator=g).to(torch.bfloat16)
+    if grow:
+        q[..., ::2] = q[..., ::2].abs()
+        kc[..., ::2] = (kc[..., ::2] * 0.1 + grow * 0.2 * torch.arange(cap)[:, None] / width).to(torch.bfloat16)
+    slots = torch.tensor([3, 0, 2])[:b]
+    sl = slots.numpy()
+    want = ov.verify_attention(npf(q), npf(kc)[sl], npf(vc)[sl], np.ones(b, np.int64), width, d ** -0.5)
+    kc[:, :, width:] = float("nan")
+    vc[:, :, width:] = float("nan")
+    say(f"prefill attention 128 width={width} contexts={b} heads={h} grow={grow}")
+    out = kernels.prefill_attention(q.to(cuda), kc.to(cuda), vc.to(cuda), slots.to(cuda), width, d ** -0.5)
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(npf(out), want, atol=BF16_TOL[0], rtol=BF16_TOL[1])
