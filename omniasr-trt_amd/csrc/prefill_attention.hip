@@ -4,6 +4,8 @@
 // b attends to keys [0, p] of its cache row; fp32 accumulation, bf16 in and out, head_dim 128, 256 or 512.
 #include <math.h>
 
+#include <algorithm>
+
 #include "attn_tiles.h"
 #include "common.h"
 
@@ -24,6 +26,7 @@ struct PrefillArgs {
   int width, H;
   float scale_log2;
   uint16_t* out;  // [B * width, H, D] bf16
+  int units8, group;  // head dim 512 in chains: heads x contexts / 8, and how many of them are listed together
 };
 
 // Workgroup -> (query block j counted from the longest, head h, context b).  The dispatcher hands consecutive
@@ -308,7 +311,7 @@ __global__ __launch_bounds__(64 * kPwWaves) __attribute__((amdgpu_waves_per_eu(2
 // (128 KB of K and V at 64 bytes a clock), 1860 of LDS; a tile takes ~3000, as a value wave issues its loads and its
 // products in one order.  The kernel this replaced added the partial scores of four 128-dimension slices through LDS,
 // with three barriers per 32 keys of 96 queries (5500 clocks for 1536 of matrix work).  Measured, 8 heads: 8 contexts
-// x 2048 521 -> 357 us (770 TFLOP/s); one context of 1433, where the longest block is the launch, 110 -> 39 us.  Tried:
+// x 2048 521 -> 357 us (770 TFLOP/s; in chains 334, see ws_group); one context of 1433, where the longest block is the launch, 110 -> 39 us.  Tried:
 // 8-byte V loads of the operand's own rows, 390 / 45 us (the memory path takes a load instruction per 64 lanes, not
 // only its bytes); the loads spread between the products, 390-430 us (the tile's rows arrive later and its products
 // compete with the scores'); K rows brought by the score waves, 404 us; wave priorities, no change.
@@ -331,111 +334,166 @@ __device__ __forceinline__ const char* scalar_pointer(const void* p) {
                                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32);
 }
 
+// Chains: a workgroup fills a CU's LDS, so with more blocks than CUs each block's start (first K tile and Q, 6-7 us)
+// and end (2-3 us) stood between the tiles of two blocks.  In a chain the next block's first tile is the tile after the
+// last: its K and V are on the way and its scores run beside the last values of the block before.  XCD x's blocks, those
+// of units (head, context) x, x + 8, .., are listed group after group of ``group`` units, within a group the longest
+// blocks first, and dealt to the XCD's kWsPerXcd workgroups there and back, so that long and short blocks even out.
+constexpr int kWsPerXcd = 32;  // workgroups at a time: one per CU
+
+// The units in a group, 0 for no chains.  Below two rounds nothing evens out (2 contexts x 1433, 1.4 rounds: 49.5 us in
+// chains, 47.9 without), nor with one unit, whose longest block is the launch (1 x 4100: 152, 146).  Two units where
+// rounds and groups then end together (block counts in 16s): few units at a time stay in the XCD's L2 (8 x 2048: 334 us,
+// 337 with 1 or 4 units, 355 with all 8, 366 without chains; 8 x 1000: 106, 105, 108, 111, 126).  Otherwise one group of
+// all (8 x 1433: 200 with 2, 192 with all, 198 without; 3 x 1433 76, without 94; 8 x 350 27, 32), up to 8 units and 256
+// blocks: with more the L2 is lost (7 x 2500, 280 blocks: 454, 444; 8 x 3000 739, 659; 16 x 1433 414, 377).
+inline int ws_group(int nqb, int units8) {
+  const int64_t blocks = (int64_t)nqb * units8;
+  if (blocks < 2 * kWsPerXcd || units8 < 2) return 0;
+  if (nqb % 16 == 0) return 2;
+  return blocks <= 256 && units8 <= 8 ? units8 : 0;
+}
+
+// A query block of a workgroup at head dim 512, its chain's ``round``-th.
+struct WsBlock {
+  int round, qb, h, b;
+};
+struct WsTile {  // key tile t of a block
+  WsBlock blk;
+  int t;
+  const char *kbase, *vbase;
+};
+
+template <bool kChain>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attn_ws_kernel(PrefillArgs a) {
   constexpr int D = kWsD;
   __shared__ __attribute__((aligned(16))) char kls[2][kWsK * kWsRow];
   __shared__ u32x4_t ps[2][2][4][64];  // [tile parity][query half][16-key step][lane]
   __shared__ float mxs[2][kWsQ];       // a tile's maxima by key half, when the reference moves
   __shared__ float als[kWsQ];          // then: the factors O is rescaled by
-  __shared__ float lsum[2][2][kWsQ];   // at the end: probability sums by key half and lane half
+  __shared__ float lsum[2][2][2][kWsQ];  // [parity of the block in the chain]: probability sums by key half, lane half
   __shared__ int moved[4];             // by tile % 4: a score passed the guard
   const int nqb = (a.width + kWsQ - 1) / kWsQ;
-  const PfBlock blk = pf_block(nqb, a.H, (int)gridDim.z);
-  const int qb = (nqb - 1 - blk.j) * kWsQ;  // the longest blocks first
-  const int h = blk.h, b = blk.b;
   const int tid = threadIdx.x, lane = tid & 63, x = lane & 31, g = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t slot = clamp64(a.slots[b], 0, a.cache_rows - 1);
-  const char* kbase = scalar_pointer(a.k + slot * a.s_row + h * a.s_head);
-  const char* vbase = scalar_pointer(a.v + slot * a.s_row + h * a.s_head);
-  const int nt = qb / kWsK + 1;  // the last tile holds the diagonal
   if (tid < 4) moved[tid] = 0;
+  // The workgroup's block of a round, from its XCD's list; false past its end.
+  auto place = [&](WsBlock& blk, int round) {
+    const int c = (int)blockIdx.x / 8;
+    const int p = round * kWsPerXcd + (round & 1 ? kWsPerXcd - 1 - c : c);
+    if (p >= a.units8 * nqb) return false;
+    const int full = a.group * nqb, g0 = p / full * a.group, r = p % full, members = min(a.group, a.units8 - g0);
+    const int unit = (g0 + r % members) * 8 + (int)blockIdx.x % 8;
+    blk = WsBlock{round, (nqb - 1 - r / members) * kWsQ, unit % a.H, unit / a.H};
+    return true;
+  };
+  auto first = [&]() {
+    WsBlock blk;
+    if constexpr (kChain) {
+      place(blk, 0);
+    } else {
+      const PfBlock one = pf_block(nqb, a.H, (int)gridDim.z);
+      blk = WsBlock{0, (nqb - 1 - one.j) * kWsQ, one.h, one.b};  // the longest blocks first
+    }
+    return blk;
+  };
+  auto next = [&](WsBlock& blk) {  // false (and blk as it was): that was the last
+    if constexpr (kChain) return place(blk, blk.round + 1);
+    return false;
+  };
 
   if (w < 4) {  // ------------------------------------------------------------------------------ scores
     const int qh = w & 1, kh = w >> 1;
-    const int query = qb + 32 * qh + x;
-    u32x4_t q[D / 16];  // q[query][16s + 8g .. + 7] (past the end the last query's: its results are not stored)
-    {
-      const uint16_t* qrow = a.q + ((int64_t)(b * a.width + min(query, a.width - 1)) * a.H + h) * D + g * 8;
-#pragma unroll
-      for (int s = 0; s < D / 16; ++s) q[s] = *reinterpret_cast<const u32x4_t*>(qrow + s * 16);
-    }
-    float m_ref = -INFINITY, thr = -INFINITY, l_run = 0.f;
     // K operands in a ring kWsAhead steps ahead of the products: an LDS read takes a few products' time to arrive.
     u32x4_t kf[kWsAhead];
     auto k_at = [&](int t, int s) {
       return *reinterpret_cast<const u32x4_t*>(&kls[t & 1][(32 * kh + x) * kWsRow + g * 16 + s * 32]);
     };
-    lds_barrier();  // the first K tile
+    WsBlock blk = first();
+    int t = 0;  // counted over the workgroup's blocks, as is all LDS
+    for (int odd = 0;; odd ^= 1) {
+      const int qb = blk.qb, query = qb + 32 * qh + x, t_last = t + qb / kWsK;  // the last tile holds the diagonal
+      u32x4_t q[D / 16];  // q[query][16s + 8g .. + 7] (past the end the last query's: its results are not stored)
+      {
+        const uint16_t* qrow = a.q + ((int64_t)(blk.b * a.width + min(query, a.width - 1)) * a.H + blk.h) * D + g * 8;
 #pragma unroll
-    for (int s = 0; s < kWsAhead; ++s) kf[s] = k_at(0, s);
-    for (int t = 0; t < nt; ++t) {
-      f32x16_t s0, s1;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s0[i] = s1[i] = 0.f;
-#pragma unroll
-      for (int s = 0; s < D / 16; ++s) {
-        if (s & 1) s1 = mfma32(kf[s % kWsAhead], q[s], s1);
-        else s0 = mfma32(kf[s % kWsAhead], q[s], s0);
-        if (s + kWsAhead < D / 16) {
-          kf[s % kWsAhead] = k_at(t, s + kWsAhead);
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one product, one LDS read
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
+        for (int s = 0; s < D / 16; ++s) q[s] = *reinterpret_cast<const u32x4_t*>(qrow + s * 16);
       }
-      float sv[16];
+      float m_ref = -INFINITY, thr = -INFINITY, l_run = 0.f;
+      if (t == 0) {
+        lds_barrier();  // the first K tile
 #pragma unroll
-      for (int i = 0; i < 16; ++i) sv[i] = s0[i] + s1[i];
-      if (t == nt - 1) {
-        const int rel = query - (t * kWsK + 32 * kh + 4 * g);  // keys 8 (i / 4) + i % 4 <= rel are seen
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sv[i] = 8 * (i >> 2) + (i & 3) <= rel ? sv[i] : -INFINITY;
+        for (int s = 0; s < kWsAhead; ++s) kf[s] = k_at(0, s);
       }
-      bool over = false;
+      for (; t <= t_last; ++t) {
+        f32x16_t s0, s1;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) over |= sv[i] > thr;
-      if (__any(over) && lane == 0) moved[t & 3] = 1;
-      float lt = 0.f;
-      auto put_p = [&](float m) {
-        lt = 0.f;
+        for (int i = 0; i < 16; ++i) s0[i] = s1[i] = 0.f;
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          u32x4_t pop;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[8 * s + 2 * e], a.scale_log2, -m));
-            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[8 * s + 2 * e + 1], a.scale_log2, -m));
-            lt += p0 + p1;
-            pop[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{p0, p1}), bf16x2_t));
+        for (int s = 0; s < D / 16; ++s) {
+          if (s & 1) s1 = mfma32(kf[s % kWsAhead], q[s], s1);
+          else s0 = mfma32(kf[s % kWsAhead], q[s], s0);
+          if (s + kWsAhead < D / 16) {
+            kf[s % kWsAhead] = k_at(t, s + kWsAhead);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one product, one LDS read
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
           }
-          ps[t & 1][qh][2 * kh + s][lane] = pop;
         }
-      };
-      put_p(m_ref == -INFINITY ? 0.f : m_ref);
-      lds_barrier();
-      const int again = moved[t & 3];  // uniform over the workgroup
+        float sv[16];
 #pragma unroll
-      for (int s = 0; s < kWsAhead; ++s) kf[s] = k_at(t + 1, s);  // (past the last tile: unused)
-      if (w == 0 && lane == 0) moved[(t + 2) & 3] = 0;
-      if (again) {
-        float mx = sv[0];
+        for (int i = 0; i < 16; ++i) sv[i] = s0[i] + s1[i];
+        if (t == t_last) {
+          const int rel = 32 * qh + x - (32 * kh + 4 * g);  // keys 8 (i / 4) + i % 4 <= rel are seen
 #pragma unroll
-        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, sv[i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-        if (g == 0) mxs[kh][32 * qh + x] = mx;
-        lds_barrier();
-        const float m_new = fmaxf(m_ref, fmaxf(mxs[0][32 * qh + x], mxs[1][32 * qh + x]) * a.scale_log2);
-        const float alpha = __builtin_amdgcn_exp2f(m_ref - (m_new == -INFINITY ? 0.f : m_new));  // m_ref = -inf: 0
-        if (kh == 0 && g == 0) als[32 * qh + x] = alpha;
-        l_run *= alpha;
-        m_ref = m_new;
-        thr = m_new == -INFINITY ? -INFINITY : (m_new + kWsGuard) / a.scale_log2;
+          for (int i = 0; i < 16; ++i) sv[i] = 8 * (i >> 2) + (i & 3) <= rel ? sv[i] : -INFINITY;
+        }
+        bool over = false;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) over |= sv[i] > thr;
+        if (__any(over) && lane == 0) moved[t & 3] = 1;
+        float lt = 0.f;
+        auto put_p = [&](float m) {
+          lt = 0.f;
+#pragma unroll
+          for (int s = 0; s < 2; ++s) {
+            u32x4_t pop;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[8 * s + 2 * e], a.scale_log2, -m));
+              const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[8 * s + 2 * e + 1], a.scale_log2, -m));
+              lt += p0 + p1;
+              pop[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{p0, p1}), bf16x2_t));
+            }
+            ps[t & 1][qh][2 * kh + s][lane] = pop;
+          }
+        };
         put_p(m_ref == -INFINITY ? 0.f : m_ref);
         lds_barrier();
+        const int again = moved[t & 3];  // uniform over the workgroup
+#pragma unroll
+        for (int s = 0; s < kWsAhead; ++s) kf[s] = k_at(t + 1, s);  // (past the last tile: unused)
+        if (w == 0 && lane == 0) moved[(t + 2) & 3] = 0;
+        if (again) {
+          float mx = sv[0];
+#pragma unroll
+          for (int i = 1; i < 16; ++i) mx = fmaxf(mx, sv[i]);
+          mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+          if (g == 0) mxs[kh][32 * qh + x] = mx;
+          lds_barrier();
+          const float m_new = fmaxf(m_ref, fmaxf(mxs[0][32 * qh + x], mxs[1][32 * qh + x]) * a.scale_log2);
+          const float alpha = __builtin_amdgcn_exp2f(m_ref - (m_new == -INFINITY ? 0.f : m_new));  // m_ref = -inf: 0
+          if (kh == 0 && g == 0) als[32 * qh + x] = alpha;
+          l_run *= alpha;
+          m_ref = m_new;
+          thr = m_new == -INFINITY ? -INFINITY : (m_new + kWsGuard) / a.scale_log2;
+          put_p(m_ref == -INFINITY ? 0.f : m_ref);
+          lds_barrier();
+        }
+        l_run += lt;
       }
-      l_run += lt;
+      lsum[odd][kh][g][32 * qh + x] = l_run;
+      if (!next(blk)) break;
     }
-    lsum[kh][g][32 * qh + x] = l_run;
     lds_barrier();
     return;
   }
@@ -452,13 +510,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int i = 0; i < 16; ++i) o[u][e][i] = 0.f;
   // K rows 16 vw .. + 15 of tile t to LDS, one row (64 lanes x 16 bytes) per load; rows past the context read its last
   // key (finite: masked).
-  const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kbase), 0, -1, 0x00020000);
-  auto bring_k = [&](int t) {
+  auto bring_k = [&](const WsTile& c, int n) {  // as tile n of the workgroup
+    const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(c.kbase), 0, -1, 0x00020000);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int key = min(t * kWsK + 16 * vw + r, a.width - 1);
+      const int key = min(c.t * kWsK + 16 * vw + r, a.width - 1);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          kr, (__attribute__((address_space(3))) void*)&kls[t & 1][(16 * vw + r) * kWsRow], 16, lane * 16,
+          kr, (__attribute__((address_space(3))) void*)&kls[n & 1][(16 * vw + r) * kWsRow], 16, lane * 16,
           (int)((uint32_t)key * (D * 2)), 0,
           0);
     }
@@ -469,12 +527,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const uint32_t vlane = (uint32_t)((8 * (x >> 4) + 4 * g) * D + 128 * vw + 8 * (x & 15)) * 2;
   const uint32_t vbytes = (uint32_t)a.width * (D * 2);
   u32x4_t v[4][4];
-  auto load_v = [&](int t, int s) {
-    const uint32_t off = (uint32_t)(t * kWsK + 16 * s) * (D * 2);
+  auto load_v = [&](const WsTile& c, int s) {
+    const uint32_t off = (uint32_t)(c.t * kWsK + 16 * s) * (D * 2);
     uint32_t used = min(off, vbytes);
     asm("" : "+s"(used));  // kept scalar (the saturating subtraction it would become is a vector instruction)
     const __amdgpu_buffer_rsrc_t vr =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vbase) + off, 0, vbytes - used, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(c.vbase) + off, 0, vbytes - used, 0x00020000);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       v[s][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(vr, vlane + j * D * 2, 0, 0));
@@ -484,9 +542,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int u = 0; u < 2; ++u) p[u][s & 1] = ps[t & 1][u][s][lane];
   };
-  // O^T += V^T P^T for tile t; ``ahead``: tile t + 1's V loads as its registers fall free.  Step s + 1's operands are
-  // built beside step s's products; the scheduler keeps each step's loads behind the permutes that read their registers.
-  auto attend_v = [&](int t, bool ahead) {
+  // O^T += V^T P^T for the workgroup's tile t; ``ahead``: the next tile's V loads as its registers fall free.  Step
+  // s + 1's operands are built beside step s's products; the scheduler keeps each step's loads behind the permutes that read their registers.
+  auto attend_v = [&](int t, const WsTile* ahead) {
     u32x4_t vop[2][4];
     auto operands = [&](int s) {
       // The lanes of a pair (u = 0, 1) hold 8 dimensions of 4 keys each; swapped, 4 dimensions (8c + 4u ..) of 8 keys:
@@ -516,7 +574,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       __builtin_amdgcn_sched_barrier(0);
-      if (ahead) load_v(t + 1, s);
+      if (ahead) load_v(*ahead, s);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -546,52 +604,90 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int i = 0; i < 16; ++i) o[u][e][i] *= al;
     }
   };
-  bring_k(0);
+  auto output = [&](const WsBlock& blk, int odd) {  // O of a finished block; then O is 0 again
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int query = blk.qb + 32 * u + x;
+      const float l = (lsum[odd][0][0][32 * u + x] + lsum[odd][0][1][32 * u + x]) +
+                      (lsum[odd][1][0][32 * u + x] + lsum[odd][1][1][32 * u + x]);
+      const float inv = l > 0.f ? 1.f / l : 1.f;
+      uint16_t* orow = a.out + ((int64_t)(blk.b * a.width + query) * a.H + blk.h) * D + 128 * vw + 32 * g;
+      auto pair = [&](float lo, float hi) {
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo * inv, hi * inv}), bf16x2_t));
+      };
+      if (query < a.width) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {  // dimensions 64r + 32g + 8i + 4k + e, k = 0, 1
+            u32x4_t out;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+              const int at = 4 * (r + 2 * k) + i;
+              out[2 * k] = pair(o[u][0][at], o[u][1][at]);
+              out[2 * k + 1] = pair(o[u][2][at], o[u][3][at]);
+            }
+            *reinterpret_cast<u32x4_t*>(orow + 64 * r + 8 * i) = out;
+          }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[u][e][i] = 0.f;
+    }
+  };
+  auto open = [&](WsTile& c) {  // the block's first tile
+    const int64_t slot = clamp64(a.slots[c.blk.b], 0, a.cache_rows - 1);
+    c.kbase = scalar_pointer(a.k + slot * a.s_row + c.blk.h * a.s_head);
+    c.vbase = scalar_pointer(a.v + slot * a.s_row + c.blk.h * a.s_head);
+    c.t = 0;
+  };
+  auto advance = [&](WsTile& c) {  // false (and c as it was): no more tiles
+    if (c.t < c.blk.qb / kWsK) {
+      ++c.t;
+      return true;
+    }
+    if (!next(c.blk)) return false;
+    open(c);
+    return true;
+  };
+  WsTile at, ahead;  // the tiles whose V and whose K come next
+  at.blk = first();
+  open(at);
+  bring_k(at, 0);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the tile is in LDS
   lds_barrier();
-  bring_k(1);
+  ahead = at;
+  bool more = advance(ahead);
+  bring_k(ahead, 1);
 #pragma unroll
-  for (int s = 0; s < 4; ++s) load_v(0, s);
+  for (int s = 0; s < 4; ++s) load_v(at, s);
   __builtin_amdgcn_s_waitcnt(0x0f70);
   lds_barrier();
   take_p(0);
-  for (int t = 1; t < nt; ++t) {  // tile t's scores, tile t - 1's values
-    bring_k(t + 1);  // unconditional (past the last tile: its last key's row, not used), so that no wait joins a branch
-    attend_v(t - 1, true);
-    // vmcnt(16): tile t + 1's K rows are in LDS, tile t's 16 V loads, issued after them, stay in flight (lds_barrier
+  int n = 1, odd = 0;
+  while (more) {  // tile n's scores, tile n - 1's values
+    const WsBlock was = at.blk;
+    at = ahead;
+    more = advance(ahead);
+    bring_k(ahead, n + 1);  // unconditional (past the last tile: that tile again, not used): no wait joins a branch
+    attend_v(n - 1, &at);
+    // vmcnt(16): tile n + 1's K rows are in LDS, tile n's 16 V loads, issued after them, stay in flight (lds_barrier
     // would wait for those too).  This wave's LDS reads of the tile are in registers by now.
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0x4f70);
     __builtin_amdgcn_s_barrier();
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    take_p(t);
+    if (kChain && at.t == 0) {
+      output(was, odd);
+      odd ^= 1;
+    }
+    take_p(n);
+    ++n;
   }
-  attend_v(nt - 1, false);
+  attend_v(n - 1, nullptr);
   lds_barrier();
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int query = qb + 32 * u + x;
-    const float l = (lsum[0][0][32 * u + x] + lsum[0][1][32 * u + x]) + (lsum[1][0][32 * u + x] + lsum[1][1][32 * u + x]);
-    const float inv = l > 0.f ? 1.f / l : 1.f;
-    if (query >= a.width) continue;
-    uint16_t* orow = a.out + ((int64_t)(b * a.width + query) * a.H + h) * D + 128 * vw + 32 * g;
-    auto pair = [&](float lo, float hi) {
-      return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo * inv, hi * inv}), bf16x2_t));
-    };
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {  // dimensions 64r + 32g + 8i + 4k + e, k = 0, 1
-        u32x4_t out;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const int at = 4 * (r + 2 * k) + i;
-          out[2 * k] = pair(o[u][0][at], o[u][1][at]);
-          out[2 * k + 1] = pair(o[u][2][at], o[u][3][at]);
-        }
-        *reinterpret_cast<u32x4_t*>(orow + 64 * r + 8 * i) = out;
-      }
-  }
+  output(at.blk, odd);
 }
 
 // Head dim 128: 256 queries per workgroup, four pairs of a score wave and a value wave (see prefill_attn_ws_kernel), each
@@ -893,8 +989,15 @@ extern "C" int omni_prefill_attention(const void* q, const void* k_cache, const 
     dim3 grid((width + omni::kPairQ - 1) / omni::kPairQ, heads, contexts);
     omni::prefill_attn_pairs_kernel<<<grid, 512, 0, s>>>(a);
   } else if (head_dim == 512) {
-    dim3 grid((width + omni::kWsQ - 1) / omni::kWsQ, heads, contexts);
-    omni::prefill_attn_ws_kernel<<<grid, 512, 0, s>>>(a);
+    const int nqb = (width + omni::kWsQ - 1) / omni::kWsQ, units = heads * contexts;
+    dim3 grid(nqb, heads, contexts);
+    a.units8 = units / 8;
+    a.group = units % 8 == 0 ? omni::ws_group(nqb, a.units8) : 0;
+    if (a.group) {
+      omni::prefill_attn_ws_kernel<true><<<8 * omni::kWsPerXcd, 512, 0, s>>>(a);
+    } else {
+      omni::prefill_attn_ws_kernel<false><<<grid, 512, 0, s>>>(a);
+    }
   } else {
     const int qw = 16 * omni::kPwSub * (omni::kPwWaves / 2);  // queries per workgroup
     dim3 grid((width + qw - 1) / qw, heads, contexts);

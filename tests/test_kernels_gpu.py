@@ -683,11 +683,13 @@ def test_verify_attention_f32_mfma(cuda, d, h, t, rows, separate):
     assert int(kernels._counters[torch.cuda.current_device()].abs().sum()) == 0
 
 
-@pytest.mark.parametrize("width,b,h", [(1, 2, 3), (63, 1, 8), (64, 3, 8), (65, 1, 1), (129, 2, 4), (333, 1, 8)])
+@pytest.mark.parametrize("width,b,h", [(1, 2, 3), (63, 1, 8), (64, 3, 8), (65, 1, 1), (129, 2, 4), (333, 1, 8),
+                                       (570, 2, 32), (700, 2, 24), (1010, 4, 8), (1000, 1, 40)])
 @pytest.mark.parametrize("grow", [0.0, 40.0])
 def test_prefill_attention_512(cuda, width, b, h, grow):
-    """The head-dim 512 prefill at the edges of its 64-query blocks and 64-key tiles, one to six tiles.  ``grow``: scores
-    that climb along the context by far more than the softmax reference's guard, so that it moves on later tiles too.
+    """The head-dim 512 prefill at the edges of its 64-query blocks and 64-key tiles, one to six tiles.  The last four
+    shapes: chains of two or more blocks per workgroup, 72, 66, 64 and 80 blocks over 32 workgroups, in one group of units
+    and in groups of two (the last of one).  ``grow``: scores that climb along the context by far more than the softmax reference's guard, so that it moves on later tiles too.
     Cache rows past the context hold NaN (stale memory): nothing of them may reach the output."""
     g = gen(512 + width + b)
     rows, cap, d = 4, -(-width // 64) * 64 + 32, 512
@@ -697,7 +699,7 @@ def test_prefill_attention_512(cuda, width, b, h, grow):
     if grow:  # the even dimensions of q positive, those of K rising with the position
         q[..., ::2] = q[..., ::2].abs()
         kc[..., ::2] = (kc[..., ::2] * 0.1 + grow * 0.1 * torch.arange(cap)[:, None] / width).to(torch.bfloat16)
-    slots = torch.tensor([3, 0, 2])[:b]
+    slots = torch.tensor([3, 0, 2, 1])[:b]
     sl = slots.numpy()
     want = ov.verify_attention(npf(q), npf(kc)[sl], npf(vc)[sl], np.ones(b, np.int64), width, d ** -0.5)
     kc[:, :, width:] = float("nan")
