@@ -235,7 +235,8 @@ __global__ __launch_bounds__(64 * kPwWaves) __attribute__((amdgpu_waves_per_eu(2
         }
         pop[u] = pex[gi][lane];
       }
-      // V operands by transpose reads, as in prefill_attn_kernel, from this wave's slice of the rows.
+      // V operands by transpose reads from this wave's slice of the rows: within 16 lanes, lane 4r + q points at key r,
+      // dimensions 4q .. + 3, and lane c receives dimension c of the four keys.
       const int rr = c >> 2, q4 = c & 3;
       const lds_char* vls = (const lds_char*)vl[t & 1];  // vl lives in LDS
 #pragma unroll
