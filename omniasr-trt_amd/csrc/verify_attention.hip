@@ -306,8 +306,11 @@ __device__ void merge_splits_fast(const AttnArgs& a, int b, int h, int nact, int
   else merge_batches<OutT, 8, 3>(a, b, h, nact, d0, dw, first_slot, gen_slot);
 }
 
-// After a split wrote its partial: the last of the row's ``nact`` splits merges them all.
-template <typename OutT>
+// After a split wrote its partial: the last of the row's ``nact`` splits merges them all.  ``kFewQueries``: with the
+// larger batches of few queries.  The vector-ALU kernel does without: with the three unrolled merges in the kernel its
+// value loop compiles to 90 instructions per load instead of 62 (bf16, 4 rows x 16 heads x 64, one query over 800-1500
+// keys: 136 us against 118).
+template <typename OutT, bool kFewQueries = true>
 __device__ __forceinline__ void finish_split(const AttnArgs& a, int b, int h, int nact) {
   if (a.separate) return;
   // This wave's partial stores (agent scope, written through) have reached the coherence point before its ticket
@@ -320,7 +323,9 @@ __device__ __forceinline__ void finish_split(const AttnArgs& a, int b, int h, in
   if (lane_id() == 0) ticket = __hip_atomic_fetch_add(counter, 1, kTicketOrder, __HIP_MEMORY_SCOPE_AGENT);
   ticket = __shfl(ticket, 0, kWave);
   if (ticket != nact - 1) return;
-  merge_splits_fast<OutT>(a, b, h, nact);  // every split's partial, read at the coherence point
+  // every split's partial, read at the coherence point
+  if constexpr (kFewQueries) merge_splits_fast<OutT>(a, b, h, nact);
+  else merge_batches<OutT, 8, 3>(a, b, h, nact, 0, -1, -1, -1);
   if (lane_id() == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -1741,7 +1746,7 @@ __global__ __launch_bounds__(64) void verify_attn_valu_kernel(AttnArgs a) {
     }
   }
   if (direct) return;
-  finish_split<Elem>(a, b, h, r.nact);
+  finish_split<Elem, false>(a, b, h, r.nact);
 }
 
 // ---------------------------------------------------------------------------------------------- combine
