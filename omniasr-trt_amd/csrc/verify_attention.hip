@@ -1753,9 +1753,10 @@ __global__ __launch_bounds__(64) void verify_attn_valu_kernel(AttnArgs a) {
 
 // Second launch of the split merge: one wave per (query row t, head, row b), every load issued at once (one
 // memory round trip).  Lane s holds split s's (m, l); each lane keeps D/64 output dimensions of every split.
+// ``early`` (see launch_combine): the first partials load beside the row's length.
 
 template <typename OutT, int DPL>
-__global__ __launch_bounds__(64) void verify_attn_combine_kernel(AttnArgs a) {
+__global__ __launch_bounds__(64) void verify_attn_combine_kernel(AttnArgs a, bool early) {
   const int t = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int lane = threadIdx.x;
   const int T = a.T, D = a.D;
@@ -1763,8 +1764,9 @@ __global__ __launch_bounds__(64) void verify_attn_combine_kernel(AttnArgs a) {
   const int d0 = has_d ? lane * DPL : 0;  // lanes past the head's dimensions read dimension 0 and store nothing
   // The partials' rows in batches of kB, every load of a batch in flight at once (slots clamped to the last one; the
   // repeats are not added), added in split order, and the partials' (m, l), lane q holding partial q's.  Plain key
-  // splits take the slots from 0 on, so the first batch and the (m, l) load beside the row's length, which says how
-  // many of them count: one memory round trip for up to kB splits.
+  // splits take the slots from 0 on, so with ``early`` the first batch and the (m, l) load beside the row's length,
+  // which says how many of them count (the others may never have been written): one memory round trip for up to kB
+  // splits.
   constexpr int kB = 16;  // one batch for up to 16 splits (the default chunk gives at most 10 at 2560 keys)
   float po[kB][DPL];
   float m, l;
@@ -1792,7 +1794,6 @@ __global__ __launch_bounds__(64) void verify_attn_combine_kernel(AttnArgs a) {
     m = a.part_ml[ml];
     l = a.part_ml[ml + 1];
   };
-  const bool early = !a.balanced && a.gen_split < 0;
   if (early) {
     load_batch(0, a.splits, a.splits - 1);
     load_ml(a.splits, a.splits - 1);
@@ -1990,10 +1991,21 @@ static int launch_attention(const AttnArgs& a, int rows, int dtype, hipStream_t 
   return omni_launch_status();
 }
 
+// Waves up to which, and partial slots of a row from which, the merge launch loads partials before it knows the row's
+// length.  A row of one split has nothing to merge, and its loads of partials nobody wrote cost 0.5 us when all rows are
+// such (12 layers of 1 row x 32 heads x 128, 60 keys: 73.7 us against 67.5), so they are left out up to 4 slots (the
+// bucket of 256 keys); with more, some row is long, and its gain covers them while the chip has room for the waves: 3
+// rows, 5 queries over 60, 60 and 500 keys 139.4 us against 141.9, one row of 1024 keys 133.3 against 136.7, 16 queries
+// over 1500 keys (512 waves) 196.3 against 198.4; but 3 rows, 11 queries over 60, 60 and 2000 keys (1056 waves) 207.4
+// against 202.2, 8 rows, 16 queries 234.2 against 215.9.
+constexpr int kEarlyMergeWaves = 512, kEarlyMergeSlots = 5;
+
 static int launch_combine(const AttnArgs& a, int rows, int dtype, hipStream_t s) {
+  const bool early = !a.balanced && a.gen_split < 0 && a.splits >= kEarlyMergeSlots &&
+                     (int64_t)rows * a.H * a.T <= kEarlyMergeWaves;
   dim3 cgrid(a.T, a.H, rows);
   const int dpl = (a.D + 63) / 64;  // output dimensions per lane
-#define OMNI_COMBINE(T_, DPL_) verify_attn_combine_kernel<T_, DPL_><<<cgrid, 64, 0, s>>>(a)
+#define OMNI_COMBINE(T_, DPL_) verify_attn_combine_kernel<T_, DPL_><<<cgrid, 64, 0, s>>>(a, early)
   if (dtype == OMNI_BF16) {
     if (dpl == 1) OMNI_COMBINE(uint16_t, 1);
     else if (dpl == 2) OMNI_COMBINE(uint16_t, 2);

@@ -747,3 +747,18 @@ def test_prefill_attention_128(cuda, width, b, h, grow):
     out = kernels.prefill_attention(q.to(cuda), kc.to(cuda), vc.to(cuda), slots.to(cuda), width, d ** -0.5)
     torch.cuda.synchronize()
     np.testing.assert_allclose(npf(out), want, atol=BF16_TOL[0], rtol=BF16_TOL[1])
+
+
+@pytest.mark.parametrize("rows,h,t,keys", [(2, 4, 5, 256), (2, 4, 5, 320), (4, 8, 16, 1024), (3, 19, 9, 1024)])
+def test_verify_attention_merge_leaves_unwritten_partials(cuda, monkeypatch, rows, h, t, keys):
+    """The merge launch on both sides of its early loads (4 and 5 slots a row; 512 and 513 waves), over short rows, empty
+    ones, full ones and rows of a few splits, in a workspace of NaN: what no split wrote reaches no output."""
+    empty = torch.empty
+
+    def nan_workspace(*size, **kw):
+        x = empty(*size, **kw)
+        return x.fill_(0xff) if kw.get("dtype") == torch.uint8 else x  # four such bytes: a NaN
+
+    monkeypatch.setattr(torch, "empty", nan_workspace)
+    lengths = torch.tensor([20, keys, 0, 130])[:rows]
+    _attn_case(cuda, torch.bfloat16, rows, h, 128, t, keys, lengths, keys, 77 + rows, BF16_TOL, chunk=64)
