@@ -523,10 +523,13 @@ struct BalancedSplit {
 // over 63 tiles: 32 41.1, 16 28.8, 8 27.6), so nt / n tiles and n T partials cost least at nt / n = sqrt(nt T / 18);
 // and no split is left with a tile less than the others (the same number of tiles each needs fewer of them).  Rows
 // that share the chip have 8 workgroups or fewer (one batch of the merge) and use them all.  Only the deal depends on
-// the result, within 1 .. wk, so approximate divisions do.
+// the result, within 1 .. wk, so approximate divisions do.  With a merge launch (fp32) a row's splits are at most its 64
+// lanes: past them one wave merges every query, partial by partial (4 heads x 128, 5 queries, 12 layers, one row of 2300
+// keys among seven of 60: 1417 us with 73 splits, 240 with 37).
 constexpr int kAllAtWork = 8;
 __device__ __forceinline__ int splits_in_use(const AttnArgs& a, int nt, int wk) {
   if (wk <= kAllAtWork) return wk;
+  if (a.separate && wk > kWave) wk = kWave;  // what the merge launch's lanes hold
   const float n = (float)nt;
   float per = ceilf(n * __builtin_amdgcn_rcpf((float)wk) - 1e-3f);
   if (!a.separate) per = fmaxf(per, rintf(__builtin_amdgcn_sqrtf(n * (float)a.T * (1.f / 18.f))));

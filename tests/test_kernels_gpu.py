@@ -762,3 +762,10 @@ def test_verify_attention_merge_leaves_unwritten_partials(cuda, monkeypatch, row
     monkeypatch.setattr(torch, "empty", nan_workspace)
     lengths = torch.tensor([20, keys, 0, 130])[:rows]
     _attn_case(cuda, torch.bfloat16, rows, h, 128, t, keys, lengths, keys, 77 + rows, BF16_TOL, chunk=64)
+
+
+@pytest.mark.parametrize("h,t", [(4, 5), (2, 1)])
+def test_verify_attention_f32_long_row(cuda, h, t):
+    """fp32, few heads: one long row among short ones is dealt more workgroups than the merge launch has lanes."""
+    lengths = torch.tensor([3, 17, 2300, 60, 0, 33, 60, 1])
+    _attn_case(cuda, torch.float32, 8, h, 128, t, 2320, lengths, 2560, 91 + h, (2e-5, 2e-5))
