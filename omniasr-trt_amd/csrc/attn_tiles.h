@@ -215,12 +215,19 @@ __device__ __forceinline__ void attend_bits(const KVTile<D>& t, const u32x4_t (&
   attend_scored<D, true>(t, sv, c_scale, st, o, g, 0, bits);
 }
 
-// A workgroup barrier ordering LDS accesses only: global loads in flight stay in flight across it (a full
-// __syncthreads waits for every outstanding memory access of the wave).
+// A workgroup barrier ordering LDS accesses only: loads into registers in flight stay in flight across it (a full
+// __syncthreads waits for every outstanding memory access of the wave).  It promises nothing for direct loads to LDS
+// (the compiler may wait for all of the wave's loads here once there are any): landed_barrier.
 __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// lds_barrier, and before it this wave's direct loads to LDS have landed: what it brought can be read after it.
+__device__ __forceinline__ void landed_barrier() {
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  lds_barrier();
 }
 
 }  // namespace omni

@@ -656,15 +656,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   at.blk = first();
   open(at);
   bring_k(at, 0);
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the tile is in LDS
-  lds_barrier();
+  landed_barrier();
   ahead = at;
   bool more = advance(ahead);
   bring_k(ahead, 1);
 #pragma unroll
   for (int s = 0; s < 4; ++s) load_v(at, s);
-  __builtin_amdgcn_s_waitcnt(0x0f70);
-  lds_barrier();
+  landed_barrier();
   take_p(0);
   int n = 1, odd = 0;
   while (more) {  // tile n's scores, tile n - 1's values
@@ -696,9 +694,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // registers) beside the softmax of tile t - 1, so its matrix and vector work overlap within the wave; value wave p
 // accumulates tile t - 2.  A pair keeps its own softmax reference (a lane's two queries see every key of the tile
 // through lanes x and x + 32), so a moved reference costs no barrier: the factors wait in LDS for the value wave.
-// K and V rows go to LDS by direct loads (score waves bring V, value waves K: neither reads what it brings, so no wait
-// for the loads comes before the barrier), 1 KB = 4 rows each, 16-byte chunks permuted within a row so that the
-// operand reads spread over the banks: chunk c of key r at position c ^ (r % 16) in K, c ^ 4 (r % 4) in V.
+// K and V rows go to LDS by direct loads (score waves bring V, value waves K: neither reads what it brings, so its
+// loads are waited for at the step's barrier alone, landed_barrier), 1 KB = 4 rows each, 16-byte chunks permuted within
+// a row so that the operand reads spread over the banks: chunk c of key r at position c ^ (r % 16) in K, c ^ 4 (r % 4)
+// in V.
 //
 // What bounds a tile (a pair's 64 queries x 64 keys): 2048 clocks of matrix work on its SIMD beside ~1900 of the score
 // wave's vector work (64 exponentials per lane at a quarter rate), one barrier per tile.  The kernel this replaced ran
@@ -846,35 +845,35 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int u = 0; u < 2; ++u) lsum[pr][g][32 * u + x] = l_run[u];
     };
     Scores sa, sb;
-    lds_barrier();  // the first K tile
+    lds_barrier();  // the first K tile (these waves have brought nothing yet)
     if (dq >= 0) step(sb, sa, 0, false);
     lds_barrier();
     int t = 1;
     for (; t + 1 <= dq; t += 2) {
       bring_v(t - 1);
       step(sa, sb, t, true);
-      lds_barrier();
+      landed_barrier();
       bring_v(t);
       step(sb, sa, t + 1, true);
-      lds_barrier();
+      landed_barrier();
     }
     if (t <= dq) {  // one more, then its scores are in sb
       bring_v(t - 1);
       step(sa, sb, t, true);
-      lds_barrier();
+      landed_barrier();
       bring_v(t);
       finish(sb, t);
-      lds_barrier();
+      landed_barrier();
       t += 2;
     } else if (dq >= 0) {
       bring_v(t - 1);
       finish(sa, t - 1);
-      lds_barrier();
+      landed_barrier();
       t += 1;
     }
     for (; t <= nt + 1; ++t) {
       if (t <= nt) bring_v(t - 1);
-      lds_barrier();
+      landed_barrier();
     }
     return;
   }
@@ -925,11 +924,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
   };
   bring_k(0);
-  lds_barrier();
+  landed_barrier();
   for (int t = 0; t <= nt + 1; ++t) {
     if (t + 1 < nt) bring_k(t + 1);
     if (t >= 2 && t - 2 <= dq) attend_v(t - 2);
-    lds_barrier();
+    landed_barrier();
   }
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
