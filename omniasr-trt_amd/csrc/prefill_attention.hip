@@ -956,6 +956,230 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
+// Head dim 128 in blocks of 192 queries, for the launches of small_blocks: one workgroup of 4 waves, two workgroups per
+// CU.  The block's 32-key tiles go through LDS once for all of its waves (double-buffered: tile t + 1's global loads are
+// in flight during tile t's math).  Each wave holds kPfSub groups of 16 queries: per tile it reads the K fragments and,
+// by LDS transpose reads, the V operands once, then runs S^T = K Q^T, the lazy softmax (causal limit as the key limit,
+// skipped on tiles the whole group sees) and O += P V for every group that sees the tile.  What bounds it is that its
+// products and its softmax share one wave: a tile takes ~1.7 times as long as in the pairs kernel, but a CU holds two.
+constexpr int kPfWaves = 4;
+constexpr int kPfSub = 3;  // 16-query groups per wave (3: 255 VGPRs, two waves per SIMD; measured fastest of 1-4)
+constexpr int kPfQueries = 16 * kPfSub * kPfWaves;
+constexpr int kPfRow = 128 * 2 + 16;  // LDS bytes per key row: 256 B of data, padded against bank conflicts
+constexpr int kPfStage = 32;          // keys per LDS stage (one barrier each), a multiple of the 32-key MFMA tile
+constexpr int kPfThreads = 64 * kPfWaves;
+constexpr int kPfChunks = kPfStage * 16 / kPfThreads;  // 16-byte chunks of K (and of V) per thread per stage
+static_assert(kPfChunks * kPfThreads == kPfStage * 16, "a stage is whole chunks per thread");
+
+// Whether a launch at head dim 128 takes blocks of 192 queries, two per CU, rather than the pairs kernel's 256, one per
+// CU: where the pairs kernel needs more than one round of its 256 workgroups and
+//  * both sizes give the same number of blocks per unit, so that this one has half the rounds, and the 192 are at most 5/6
+//    full on the mean (past that its time grows with the queries, the pairs kernel's does not);
+//  * or, with one block more per unit at two or four blocks of 256, the pairs kernel's last round is nearly empty and this
+//    kernel takes fewer rounds (with three, the blocks of that round are the short ones, and it costs little).
+// Pairs kernel / this one, us: 160 units (5 contexts x 32 heads) x 257 27.3 / 22.7, x 300 27.4 / 24.8, x 385 33.5 / 30.6, x 384
+// 30.0 / 32.2 (full: pairs); 256 x 257 29.0 / 24.2; 320 x 129 22.0 / 18.8; 130 x 512 40.7 / 32.9, 192 x 512 42.2 / 48.3
+// (as many rounds: pairs); 96 x 800 50.8 / 47.0, 96 x 640 35.4 / 41.5 (three blocks: pairs).
+inline bool small_blocks(int width, int64_t units) {
+  constexpr int kCus = 256;
+  const int n = (width + kPairQ - 1) / kPairQ, small = (width + kPfQueries - 1) / kPfQueries;
+  const int64_t blocks = n * units, rounds = (blocks + kCus - 1) / kCus;
+  if (rounds < 2) return false;
+  if (n == small) return width <= kPfQueries * 5 / 6 * n;
+  const int64_t small_rounds = (small * units + 2 * kCus - 1) / (2 * kCus), last = blocks % kCus;
+  if (small != n + 1 || (n != 2 && n != 4) || last == 0 || small_rounds >= rounds) return false;
+  return last <= 96 || (2 * small_rounds <= rounds && last <= 128);
+}
+
+// The softmax step of one 16-query group for one tile: mask (key0 + j >= lim), lazy reference max, this lane's
+// 8 probabilities packed as the P operand.  (The same arithmetic as attend().)
+template <int NB>
+__device__ __forceinline__ u32x4_t softmax_tile(float (&sv)[8], float c_scale, SoftmaxState& st, f32x4_t (&o)[NB],
+                                                int g, int key0, int lim, bool whole) {
+  bool over = false;
+  if (!whole) {  // whole (wave-uniform): every query of the group sees every key of the tile
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sv[j] = key0 + j < lim ? sv[j] : -INFINITY;
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) over |= sv[j] > st.thr;
+  if (__any(over)) {
+    float mx = sv[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) mx = fmaxf(mx, sv[j]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    const float m_new = fmaxf(st.m_ref, mx * c_scale);
+    rescale<NB>(st.m_ref, m_new == -INFINITY ? 0.f : m_new, st.l_run, o, g);
+    st.m_ref = m_new;
+    st.thr = m_new == -INFINITY ? -INFINITY : (m_new + kLazyLog2) / c_scale;
+  }
+  const float m_use = st.m_ref == -INFINITY ? 0.f : st.m_ref;
+  float p[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    p[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[j], c_scale, -m_use));
+    st.l_run += p[j];
+  }
+  u32x4_t pop;
+#pragma unroll
+  for (int w = 0; w < 4; ++w)
+    pop[w] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{p[2 * w], p[2 * w + 1]}), bf16x2_t));
+  return pop;
+}
+
+__global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attn_kernel(
+    PrefillArgs a) {
+  constexpr int D = 128, KS = D / 32;
+  __shared__ __attribute__((aligned(16))) char lds[2][2][kPfStage * kPfRow];  // [buffer][K, V][key rows]
+  const int nqb = (a.width + kPfQueries - 1) / kPfQueries;
+  const PfBlock blk = pf_block(nqb, a.H, (int)gridDim.z);
+  const int qb = (nqb - 1 - blk.j) * kPfQueries;  // the longest blocks first
+  const int h = blk.h, b = blk.b;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t slot = clamp64(a.slots[b], 0, a.cache_rows - 1);
+  const uint16_t* kbase = a.k + slot * a.s_row + h * a.s_head;
+  const uint16_t* vbase = a.v + slot * a.s_row + h * a.s_head;
+  const int kend = min(qb + kPfQueries, a.width);  // keys the block's last query sees
+  const int nt = (kend + kPfStage - 1) / kPfStage;
+
+  // Global -> LDS: thread tid moves 16-byte chunks tid, tid + kPfThreads, ... of the stage's K and of its V (kPfStage rows x
+  // 256 B each).  Rows past the context read its last key (finite: masked by the causal limit, never NaN).
+  u32x4_t stage[2 * kPfChunks];
+  auto fetch = [&](int t) {
+#pragma unroll
+    for (int e = 0; e < kPfChunks; ++e) {
+      const int ci = tid + e * kPfThreads, r = ci >> 4, col = ci & 15;
+      const int key = min(t * kPfStage + r, a.width - 1);
+      stage[e] = *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)key * D + col * 8);
+      stage[kPfChunks + e] = *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)key * D + col * 8);
+    }
+  };
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int e = 0; e < kPfChunks; ++e) {
+      const int ci = tid + e * kPfThreads, r = ci >> 4, col = ci & 15;
+      *reinterpret_cast<u32x4_t*>(&lds[buf][0][r * kPfRow + col * 16]) = stage[e];
+      *reinterpret_cast<u32x4_t*>(&lds[buf][1][r * kPfRow + col * 16]) = stage[kPfChunks + e];
+    }
+  };
+
+  // The wave's groups: queries q0[u] + c, u < kPfSub (group u of wave w: block rows 16 (w + kPfWaves u)).
+  int q0[kPfSub];
+  u32x4_t qop[kPfSub][KS];  // B operand of S^T = K Q^T: lane (c, g) holds q[q0 + c][32s + 8g .. +7] (0 past the end)
+  SoftmaxState st[kPfSub];
+  f32x4_t o[kPfSub][D / 16];
+#pragma unroll
+  for (int u = 0; u < kPfSub; ++u) {
+    q0[u] = qb + 16 * (w + kPfWaves * u);
+    const bool live = q0[u] + c < a.width;
+    const uint16_t* qrow = a.q + ((int64_t)(b * a.width + (live ? q0[u] + c : 0)) * a.H + h) * D + g * 8;
+#pragma unroll
+    for (int s2 = 0; s2 < KS; ++s2)
+      qop[u][s2] = live ? *reinterpret_cast<const u32x4_t*>(qrow + s2 * 32) : u32x4_t{0u, 0u, 0u, 0u};
+    st[u] = SoftmaxState{-INFINITY, -INFINITY, 0.f};
+#pragma unroll
+    for (int nb = 0; nb < D / 16; ++nb) o[u][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+
+  fetch(0);
+  put(0);
+  __syncthreads();
+  for (int t = 0; t < nt; ++t) {
+    fetch(t + 1 < nt ? t + 1 : t);  // unconditional: the last iteration re-reads its own tile (cache hit)
+    // The stage's 32-key MFMA tiles in turn.
+#pragma unroll
+    for (int sub = 0; sub < kPfStage / 32; ++sub) {
+    const int key0 = t * kPfStage + sub * 32;
+    // Groups that see the tile (wave-uniform): a live group whose last query reaches the tile's first key.
+    bool act[kPfSub];
+    bool any = false;
+#pragma unroll
+    for (int u = 0; u < kPfSub; ++u) {
+      act[u] = q0[u] < a.width && key0 <= q0[u] + 15;
+      any |= act[u];
+    }
+    if (any) {
+      const char* kl = lds[t & 1][0] + sub * 32 * kPfRow;
+      const char* vl = lds[t & 1][1] + sub * 32 * kPfRow;
+      u32x4_t pop[kPfSub];
+      {
+        u32x4_t kf[2][KS];
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb) {
+          const int rk = 8 * (c >> 2) + 4 * mb + (c & 3);
+#pragma unroll
+          for (int s2 = 0; s2 < KS; ++s2) kf[mb][s2] = *reinterpret_cast<const u32x4_t*>(kl + rk * kPfRow + g * 16 + s2 * 64);
+        }
+#pragma unroll
+        for (int u = 0; u < kPfSub; ++u) {
+          if (!act[u]) continue;
+          f32x4_t sacc[2];
+#pragma unroll
+          for (int mb = 0; mb < 2; ++mb) {
+            sacc[mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s2 = 0; s2 < KS; ++s2)
+              sacc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[mb][s2]),
+                                                                 __builtin_bit_cast(bf16x8_t, qop[u][s2]), sacc[mb],
+                                                                 0, 0, 0);
+          }
+          float sv[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) sv[j] = sacc[j >> 2][j & 3];
+          pop[u] = softmax_tile<D / 16>(sv, a.scale_log2, st[u], o[u], g, key0 + 8 * g, q0[u] + c + 1,
+                                        key0 + 31 <= q0[u]);
+        }
+      }
+      {
+        // V operands by transpose reads: in lane group g (keys 8g .. 8g + 7) lane 4r + q points at key
+        // 8g + 4h + r, dimensions 16e + 4q .. 16e + 4q + 3 (h = 0, 1), and ds_read_b64_tr_b16 hands lane c the
+        // four keys' dimension 16e + c: block e's B operand, output column c = dimension 16e + c.
+        const int rr = c >> 2, q4 = c & 3;
+        const lds_char* vls = (const lds_char*)vl;  // vl points into LDS
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int off = (8 * g + rr) * kPfRow + (16 * e + 4 * q4) * 2;
+          const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vls + off));
+          const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vls + off + 4 * kPfRow));
+          u32x4_t bop;
+          bop[0] = (uint32_t)(uint16_t)lo[0] | ((uint32_t)(uint16_t)lo[1] << 16);
+          bop[1] = (uint32_t)(uint16_t)lo[2] | ((uint32_t)(uint16_t)lo[3] << 16);
+          bop[2] = (uint32_t)(uint16_t)hi[0] | ((uint32_t)(uint16_t)hi[1] << 16);
+          bop[3] = (uint32_t)(uint16_t)hi[2] | ((uint32_t)(uint16_t)hi[3] << 16);
+#pragma unroll
+          for (int u = 0; u < kPfSub; ++u) {
+            if (!act[u]) continue;
+            o[u][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, pop[u]),
+                                                              __builtin_bit_cast(bf16x8_t, bop), o[u][e], 0, 0, 0);
+          }
+        }
+      }
+    }
+    }
+    put((t + 1) & 1);
+    __syncthreads();
+  }
+
+  // ---- each group's 16 output rows: O / l, rounded to bf16
+#pragma unroll
+  for (int u = 0; u < kPfSub; ++u) {
+    float l_tot = st[u].l_run + __shfl_xor(st[u].l_run, 16, kWave);
+    l_tot += __shfl_xor(l_tot, 32, kWave);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float li = __shfl(l_tot, 4 * g + i, kWave);
+      const int qq = q0[u] + 4 * g + i;
+      if (qq >= a.width) continue;
+      const float div = li > 0.f ? li : 1.f;
+      uint16_t* orow = a.out + ((int64_t)(b * a.width + qq) * a.H + h) * D;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) orow[16 * e + c] = (uint16_t)pack_bf16x2(o[u][e][i] / div, 0.f);  // dim 16e + c
+    }
+  }
+}
+
 }  // namespace omni
 
 extern "C" int omni_prefill_attention(const void* q, const void* k_cache, const void* v_cache, int64_t stride_row,
@@ -986,8 +1210,13 @@ extern "C" int omni_prefill_attention(const void* q, const void* k_cache, const 
   a.out = (uint16_t*)out;
   hipStream_t s = (hipStream_t)stream;
   if (head_dim == 128) {
-    dim3 grid((width + omni::kPairQ - 1) / omni::kPairQ, heads, contexts);
-    omni::prefill_attn_pairs_kernel<<<grid, 512, 0, s>>>(a);
+    if (omni::small_blocks(width, (int64_t)heads * contexts)) {
+      dim3 grid((width + omni::kPfQueries - 1) / omni::kPfQueries, heads, contexts);
+      omni::prefill_attn_kernel<<<grid, omni::kPfThreads, 0, s>>>(a);
+    } else {
+      dim3 grid((width + omni::kPairQ - 1) / omni::kPairQ, heads, contexts);
+      omni::prefill_attn_pairs_kernel<<<grid, 512, 0, s>>>(a);
+    }
   } else if (head_dim == 512) {
     const int nqb = (width + omni::kWsQ - 1) / omni::kWsQ, units = heads * contexts;
     dim3 grid(nqb, heads, contexts);

@@ -749,6 +749,38 @@ def test_prefill_attention_128(cuda, width, b, h, grow):
     np.testing.assert_allclose(npf(out), want, atol=BF16_TOL[0], rtol=BF16_TOL[1])
 
 
+def _prefill_sampled(cuda, width, b, h, d):
+    """The prefill of many blocks against float32 attention of one query per 64 (and the last) of every context and head:
+    every block of a launch is looked at.  Cache rows in another order than the contexts, NaN past each context."""
+    g = torch.Generator(device=cuda).manual_seed(31 * width + b)
+    rows, cap = b + 2, -(-width // 64) * 64 + 32
+    normal = lambda *shape: torch.empty(shape, device=cuda, dtype=torch.bfloat16).normal_(generator=g)
+    q, kc, vc = normal(b * width, h, d), normal(rows, h, cap, d), normal(rows, h, cap, d)
+    slots = torch.randperm(rows, generator=gen(width))[:b]
+    kc[:, :, width:] = float("nan")
+    vc[:, :, width:] = float("nan")
+    say(f"prefill attention sampled d={d} width={width} contexts={b} heads={h}")
+    out = kernels.prefill_attention(q, kc, vc, slots.to(cuda), width, d ** -0.5)
+    torch.cuda.synchronize()
+    at = torch.arange(0, width, 64)
+    at = torch.cat([torch.minimum(at + torch.randint(0, 64, at.shape, generator=gen(b)), torch.tensor(width - 1)),
+                    torch.tensor([width - 1])])
+    dead = torch.arange(width)[None] > at[:, None]
+    out, q = (x.view(b, width, h, d)[:, at.to(cuda)].cpu().float() for x in (out, q))
+    for c in range(b):
+        k, v = (x[int(slots[c]), :, :width].cpu().float() for x in (kc, vc))
+        scores = (q[c].transpose(0, 1) @ k.transpose(1, 2)) * d ** -0.5
+        want = torch.softmax(scores.masked_fill(dead, float("-inf")), -1) @ v
+        np.testing.assert_allclose(out[c].transpose(0, 1).numpy(), want.numpy(), atol=BF16_TOL[0], rtol=BF16_TOL[1])
+
+
+@pytest.mark.parametrize("width,b,h", [(70, 4, 66), (160, 8, 33), (161, 8, 33), (257, 2, 68), (257, 8, 32), (320, 2, 65),
+                                       (321, 2, 65), (385, 2, 65), (512, 2, 65), (512, 2, 88), (800, 3, 32), (961, 3, 32)])
+def test_prefill_attention_128_many_blocks(cuda, width, b, h):
+    """Head dim 128 in more than 256 blocks of 256 queries, on both sides of the rule between them and blocks of 192."""
+    _prefill_sampled(cuda, width, b, h, 128)
+
+
 @pytest.mark.parametrize("rows,h,t,keys", [(2, 4, 5, 256), (2, 4, 5, 320), (4, 8, 16, 1024), (3, 19, 9, 1024)])
 def test_verify_attention_merge_leaves_unwritten_partials(cuda, monkeypatch, rows, h, t, keys):
     """The merge launch on both sides of its early loads (4 and 5 slots a row; 512 and 513 waves), over short rows, empty
