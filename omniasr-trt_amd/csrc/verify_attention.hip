@@ -516,24 +516,54 @@ struct BalancedSplit {
   int b, k, nact, first;
 };
 
-// Splits that work on a row of ``nt`` tiles dealt ``wk`` workgroups.  The row's last split reads every partial (T x D
-// floats each) through one CU, so a row alone on the chip is done sooner with fewer splits of more tiles: measured at 1
-// row x 8 heads x 512, a tile of a split costs ~1.5 us and a partial ~0.08 us per query (45 tiles, 5 queries: 32
-// splits 20.1 us, 23 18.1, 15 16.3, 12 16.7, 8 18.1; 9 queries over 16 tiles: 16 splits 19.0 us, 8 14.4; 16 queries
-// over 63 tiles: 32 41.1, 16 28.8, 8 27.6), so nt / n tiles and n T partials cost least at nt / n = sqrt(nt T / 18);
-// and no split is left with a tile less than the others (the same number of tiles each needs fewer of them).  Rows
-// that share the chip have 8 workgroups or fewer (one batch of the merge) and use them all.  Only the deal depends on
-// the result, within 1 .. wk, so approximate divisions do.  With a merge launch (fp32) a row's splits are at most its 64
-// lanes: past them one wave merges every query, partial by partial (4 heads x 128, 5 queries, 12 layers, one row of 2300
-// keys among seven of 60: 1417 us with 73 splits, 240 with 37).
+// Approximately the quotient rounded up (exact for the sizes of a deal; only speed rests on it).
+__device__ __forceinline__ float tiles_up(float n, float by) { return ceilf(n * __builtin_amdgcn_rcpf(by) - 1e-3f); }
+
+// Splits that work on a row of ``nt`` tiles dealt ``wk`` workgroups; at most 8 (one batch of the merge) are all at work.
+// The row's last split reads every partial through one CU, batch after batch of merge_splits_fast, so a row with many
+// workgroups (alone on the chip, one long row among short ones, or few heads) is done sooner with fewer splits of more
+// tiles.  Measured, head dim 512: a tile of a split takes 1.5 us and a batch 1.1 to 1.6 us per kR x 256 floats of a
+// wave's T x 128 (1 row x 8 heads, 10 tiles, 16 queries: 8 splits 17 us, 9 21); a head dim of 256 halves the tile alone.
+// In units of 0.75 us: D / 256 per tile, 1.5 per batch and pass, and 0.1 per query for each partial within a batch.
+// Three candidates are weighed: the splits that balance tiles against partials in flight (nt / n = sqrt(nt T / 18)), one
+// batch less, and that batch full, each with no more splits than its number of tiles needs.
+// Measured over 1 to 16 rows of 300 to 2300 keys, even and ragged, T = 1 to 32, 4 to 16 heads of 256 and 512: within 1.8%
+// of the best number of splits on the mean and at most 4% slower than all at work (5 queries, 8 heads x 256, one long row
+// of 16), which is 26% off on the mean (the first candidate alone: 4.4%, and up to 6% slower than all at work).  12 layers, 8 heads x 512, 16 queries, one row of 2300
+// keys among fifteen of 40: 12 splits (all) 400 us, 9 (the first candidate) 416, 8 381; 16 x 256, one row of 2300: 16 splits
+// 311 us, 9 304, 8 260.
+// With a merge launch (fp32) a row's splits are at most its 64 lanes: past them one wave merges every query, partial by
+// partial (4 heads x 128, 5 queries, 12 layers, one row of 2300 keys among seven of 60: 1417 us with 73 splits, 240 with
+// 37).  The result is within 1 .. wk.
 constexpr int kAllAtWork = 8;
 __device__ __forceinline__ int splits_in_use(const AttnArgs& a, int nt, int wk) {
   if (wk <= kAllAtWork) return wk;
   if (a.separate && wk > kWave) wk = kWave;  // what the merge launch's lanes hold
-  const float n = (float)nt;
-  float per = ceilf(n * __builtin_amdgcn_rcpf((float)wk) - 1e-3f);
-  if (!a.separate) per = fmaxf(per, rintf(__builtin_amdgcn_sqrtf(n * (float)a.T * (1.f / 18.f))));
-  const int use = (int)ceilf(n * __builtin_amdgcn_rcpf(fmaxf(per, 1.f)) - 1e-3f);
+  const float n = (float)(nt > 0 ? nt : 1), all = (float)wk;
+  float per = fmaxf(tiles_up(n, all), 1.f), best = 0.f;
+  if (a.separate) {
+    best = tiles_up(n, per);
+  } else {
+    const float T = (float)a.T, tile = (float)a.D * (1.f / 256.f);
+    const int nf = a.T * 128;
+    const float batch = nf <= 256 ? 32.f : nf <= 512 ? 16.f : 8.f;  // merge_splits_fast's
+    const float pass = nf <= 512 ? 1.5f : 1.5f * (float)((nf + 767) / 768);
+    per = fmaxf(per, rintf(__builtin_amdgcn_sqrtf(n * T * (1.f / 18.f))));
+    const float first = tiles_up(n, per), batches = tiles_up(first, batch);
+    float least = INFINITY;
+    auto weigh = [&](float splits) {
+      const float tiles = fmaxf(tiles_up(n, fminf(splits, all)), 1.f), s = tiles_up(n, tiles);
+      const float cost = tile * tiles + pass * tiles_up(s, batch) + 0.1f * T * s;
+      if (cost < least) {
+        least = cost;
+        best = s;
+      }
+    };
+    weigh(first);
+    weigh(fmaxf((batches - 1.f) * batch, 8.f));
+    weigh(batches * batch);
+  }
+  const int use = (int)best;
   return use < 1 ? 1 : use > wk ? wk : use;
 }
 

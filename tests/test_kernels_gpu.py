@@ -801,3 +801,14 @@ def test_verify_attention_f32_long_row(cuda, h, t):
     """fp32, few heads: one long row among short ones is dealt more workgroups than the merge launch has lanes."""
     lengths = torch.tensor([3, 17, 2300, 60, 0, 33, 60, 1])
     _attn_case(cuda, torch.float32, 8, h, 128, t, 2320, lengths, 2560, 91 + h, (2e-5, 2e-5))
+
+
+@pytest.mark.parametrize("h,d,t,rest", [(8, 512, 16, 15), (8, 512, 1, 7), (8, 512, 3, 2), (8, 256, 9, 3), (16, 256, 16, 1),
+                                        (16, 256, 5, 7), (4, 512, 32, 3), (2, 256, 2, 5), (1, 512, 9, 1)])
+def test_verify_attention_wide_long_row(cuda, h, d, t, rest):
+    """Wide heads, one long row among short ones: dealt more than 8 workgroups, it puts as many of them to work as one,
+    two or more batches of the merge hold, by queries and head dim.  The tickets are left zero."""
+    for n in (2300, 1000, 257):
+        lengths = torch.tensor([40 + 3 * i for i in range(rest)] + [n])
+        _attn_case(cuda, torch.bfloat16, rest + 1, h, d, t, 2336, lengths, 2336, 31 + n + t, BF16_TOL)
+    assert int(kernels._counters[torch.cuda.current_device()].abs().sum()) == 0
