@@ -342,17 +342,56 @@ __device__ __forceinline__ const char* scalar_pointer(const void* p) {
 // blocks first, and dealt to the XCD's kWsPerXcd workgroups there and back, so that long and short blocks even out.
 constexpr int kWsPerXcd = 32;  // workgroups at a time: one per CU
 
-// The units in a group, 0 for no chains.  Below two rounds nothing evens out (2 contexts x 1433, 1.4 rounds: 49.5 us in
-// chains, 47.9 without), nor with one unit, whose longest block is the launch (1 x 4100: 152, 146).  Two units where
-// rounds and groups then end together (block counts in 16s): few units at a time stay in the XCD's L2 (8 x 2048: 334 us,
-// 337 with 1 or 4 units, 355 with all 8, 366 without chains; 8 x 1000: 106, 105, 108, 111, 126).  Otherwise one group of
-// all (8 x 1433: 200 with 2, 192 with all, 198 without; 3 x 1433 76, without 94; 8 x 350 27, 32), up to 8 units and 256
-// blocks: with more the L2 is lost (7 x 2500, 280 blocks: 454, 444; 8 x 3000 739, 659; 16 x 1433 414, 377).
+// The longest chain of an XCD's workgroups, in tiles (and one for each block), with ``group`` units listed together: the
+// deal of prefill_attn_ws_kernel's ``place``, block after block.
+inline int ws_longest(int nqb, int units8, int group) {
+  int tiles[kWsPerXcd] = {}, c = 0, step = 1;
+  for (int g0 = 0; g0 < units8; g0 += group) {
+    const int members = std::min(group, units8 - g0);
+    for (int t = nqb; t > 0; --t) {
+      for (int m = 0; m < members; ++m) {
+        tiles[c] += t + 1;
+        c += step;
+        if (c == kWsPerXcd || c < 0) {  // there and back: the end's workgroup takes two in a row
+          step = -step;
+          c += step;
+        }
+      }
+    }
+  }
+  return *std::max_element(tiles, tiles + kWsPerXcd);
+}
+
+// The units in a group, 0 for no chains: what is predicted to end first, in tiles.
+//  * No chains: an even share of the XCD's tiles and two for each block's start and end, and nqb / 4 for what the last
+//    blocks leave idle.
+//  * Groups of up to 8 units, or one of all: the longest chain of the deal (whether groups end with a round decides: at
+//    8 x 1433 two units at a time take 201 us, all 193, no chains 199, at 8 x 1536 199, 209 and 228), 0.1% longer for each
+//    block of a group past 128, whose K and V the XCD's L2 no longer holds (16 x 1024, even chains all: 214 us with 2
+//    units, 225 with 8, 253 with 16), and 2% for a unit alone (8 x 2048 336, with 2 330).
+// Below two rounds nothing evens out (2 contexts x 1433, 1.4 rounds: 49.5 us in chains, 47.9 without), nor with one unit,
+// whose longest block is the launch (1 x 4100: 152, 146).
+// Measured at 103 shapes, 8 heads, 2 to 16 contexts x 330 to 3000, every group size: the choice is within 1% of the best
+// one on the mean, 14% at most (16 x 640, 126 us against 111).  us, 8 contexts x width, without chains / in the chosen
+// groups: 500 42 / 37, 1984 317 (none chosen; 343 with all 8), 2048 360 / 330, 2049 369 / 354, 2300 432 / 398, 2560 507 /
+// 488, 3000 640 (none); 5 x 1024 84 / 74; 12 x 500 78 / 64; 16 x 1536 443 / 391.  The choice takes the host ~2 ns for each
+// block of each candidate.
 inline int ws_group(int nqb, int units8) {
-  const int64_t blocks = (int64_t)nqb * units8;
-  if (blocks < 2 * kWsPerXcd || units8 < 2) return 0;
-  if (nqb % 16 == 0) return 2;
-  return blocks <= 256 && units8 <= 8 ? units8 : 0;
+  if ((int64_t)nqb * units8 < 2 * kWsPerXcd || units8 < 2) return 0;
+  const float n = (float)nqb;
+  float least = (float)units8 * n * ((n + 1.f) * 0.5f + 2.f) / kWsPerXcd + 0.25f * n;
+  int pick = 0;
+  for (int i = 1; i <= std::min(units8, 9); ++i) {
+    const int group = i == 9 ? units8 : i;
+    const float spilled = (float)std::max((int64_t)group * nqb - 128, (int64_t)0);
+    const float tiles =
+        (float)ws_longest(nqb, units8, group) * (1.f + 0.001f * spilled) * (group == 1 ? 1.02f : 1.f);
+    if (tiles < least) {
+      least = tiles;
+      pick = group;
+    }
+  }
+  return pick;
 }
 
 // A query block of a workgroup at head dim 512, its chain's ``round``-th.

@@ -781,6 +781,14 @@ def test_prefill_attention_128_many_blocks(cuda, width, b, h):
     _prefill_sampled(cuda, width, b, h, 128)
 
 
+@pytest.mark.parametrize("width,b,h", [(640, 8, 8), (1020, 5, 8), (1500, 8, 8), (1984, 8, 8), (2010, 5, 8), (2300, 8, 8),
+                                       (500, 12, 8)])
+def test_prefill_attention_512_long_chains(cuda, width, b, h):
+    """Head dim 512, chains of up to nine blocks per workgroup over up to four groups of units, the last group whole or
+    not, and none."""
+    _prefill_sampled(cuda, width, b, h, 512)
+
+
 @pytest.mark.parametrize("rows,h,t,keys", [(2, 4, 5, 256), (2, 4, 5, 320), (4, 8, 16, 1024), (3, 19, 9, 1024)])
 def test_verify_attention_merge_leaves_unwritten_partials(cuda, monkeypatch, rows, h, t, keys):
     """The merge launch on both sides of its early loads (4 and 5 slots a row; 512 and 513 waves), over short rows, empty
