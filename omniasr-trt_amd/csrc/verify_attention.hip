@@ -493,9 +493,9 @@ __device__ __forceinline__ int gen_count(const AttnArgs& a, int64_t row) {
   return (int)clamp64(a.gen_len[row], 0, a.gen_cap);
 }
 
-// The generated keys in use, into LDS, every load in one round trip (the caller's barrier follows): with the step's list
-// only each group's count, gl[group T]; otherwise every beam's, gl[row].  A group's thread reads its own list count back
-// (gen_keys) without a barrier.
+// The generated keys in use, into LDS, every load in one round trip (the caller's barrier follows): with the step's
+// list only each group's count, gl[group T]; otherwise every beam's, gl[row].  A group's thread reads its own list count
+// back (gen_keys) without a barrier.
 __device__ __forceinline__ void load_gen_counts(const AttnArgs& a, int groups, int* gl, int nt) {
   if (a.glist) {
     for (int g = threadIdx.x; g < groups; g += nt) gl[g * a.T] = min(a.gcount[g], a.gen_table);  // at most the table
@@ -522,19 +522,20 @@ __device__ __forceinline__ float tiles_up(float n, float by) { return ceilf(n * 
 // Splits that work on a row of ``nt`` tiles dealt ``wk`` workgroups; at most 8 (one batch of the merge) are all at work.
 // The row's last split reads every partial through one CU, batch after batch of merge_splits_fast, so a row with many
 // workgroups (alone on the chip, one long row among short ones, or few heads) is done sooner with fewer splits of more
-// tiles.  Measured, head dim 512: a tile of a split takes 1.5 us and a batch 1.1 to 1.6 us per kR x 256 floats of a
-// wave's T x 128 (1 row x 8 heads, 10 tiles, 16 queries: 8 splits 17 us, 9 21); a head dim of 256 halves the tile alone.
-// In units of 0.75 us: D / 256 per tile, 1.5 per batch and pass, and 0.1 per query for each partial within a batch.
-// Three candidates are weighed: the splits that balance tiles against partials in flight (nt / n = sqrt(nt T / 18)), one
-// batch less, and that batch full, each with no more splits than its number of tiles needs.
+// tiles: the number that balances tiles against partials in flight, nt / n = sqrt(nt T / 18).  Where those take more
+// than one batch, they are weighed against one batch less and against the last batch full.  Measured, head dim 512: a
+// tile of a split takes 1.5 us and a batch 1.1 to 1.6 us per kR x 256 floats of a wave's T x 128 (1 row x 8 heads, 10
+// tiles, 16 queries: 8 splits 17 us, 9 21); a head dim of 256 halves the tile alone.  So in units of 0.75 us: D / 256 per
+// tile, 1.5 per batch and pass, and 0.1 per query for each partial within a batch; no candidate has more splits than its
+// number of tiles needs.
 // Measured over 1 to 16 rows of 300 to 2300 keys, even and ragged, T = 1 to 32, 4 to 16 heads of 256 and 512: within 1.8%
-// of the best number of splits on the mean and at most 4% slower than all at work (5 queries, 8 heads x 256, one long row
-// of 16), which is 26% off on the mean (the first candidate alone: 4.4%, and up to 6% slower than all at work).  12 layers, 8 heads x 512, 16 queries, one row of 2300
-// keys among fifteen of 40: 12 splits (all) 400 us, 9 (the first candidate) 416, 8 381; 16 x 256, one row of 2300: 16 splits
-// 311 us, 9 304, 8 260.
+// of the best number of splits on the mean and at most 4% slower than all at work (5 queries, 8 heads x 256, one long
+// row of 16), which is 26% off on the mean (the balance alone: 4.4%, and up to 6% slower than all at work).  12 layers, 8
+// heads x 512, 16 queries, one row of 2300 keys among fifteen of 40: 12 splits (all) 400 us, 9 (the balance) 416, 8 381;
+// 16 x 256, one row of 2300: 16 splits 311 us, 9 304, 8 260.
 // With a merge launch (fp32) a row's splits are at most its 64 lanes: past them one wave merges every query, partial by
-// partial (4 heads x 128, 5 queries, 12 layers, one row of 2300 keys among seven of 60: 1417 us with 73 splits, 240 with
-// 37).  The result is within 1 .. wk.
+// partial (4 heads x 128, 5 queries, 12 layers, one row of 2300 keys among seven of 60: 1417 us with 73 splits, 240
+// with 37).  The result is within 1 .. wk.
 constexpr int kAllAtWork = 8;
 __device__ __forceinline__ int splits_in_use(const AttnArgs& a, int nt, int wk) {
   if (wk <= kAllAtWork) return wk;
@@ -548,9 +549,9 @@ __device__ __forceinline__ int splits_in_use(const AttnArgs& a, int nt, int wk) 
     const int nf = a.T * 128;
     const float batch = nf <= 256 ? 32.f : nf <= 512 ? 16.f : 8.f;  // merge_splits_fast's
     const float pass = nf <= 512 ? 1.5f : 1.5f * (float)((nf + 767) / 768);
-    per = fmaxf(per, rintf(__builtin_amdgcn_sqrtf(n * T * (1.f / 18.f))));
-    const float first = tiles_up(n, per), batches = tiles_up(first, batch);
     float least = INFINITY;
+    per = fmaxf(per, rintf(__builtin_amdgcn_sqrtf(n * T * (1.f / 18.f))));
+    best = tiles_up(n, per);
     auto weigh = [&](float splits) {
       const float tiles = fmaxf(tiles_up(n, fminf(splits, all)), 1.f), s = tiles_up(n, tiles);
       const float cost = tile * tiles + pass * tiles_up(s, batch) + 0.1f * T * s;
@@ -559,9 +560,12 @@ __device__ __forceinline__ int splits_in_use(const AttnArgs& a, int nt, int wk) 
         best = s;
       }
     };
-    weigh(first);
-    weigh(fmaxf((batches - 1.f) * batch, 8.f));
-    weigh(batches * batch);
+    if (best > batch) {
+      const float batches = tiles_up(best, batch);
+      weigh(best);
+      weigh((batches - 1.f) * batch);
+      weigh(batches * batch);
+    }
   }
   const int use = (int)best;
   return use < 1 ? 1 : use > wk ? wk : use;
