@@ -231,9 +231,11 @@ int omni_beam_attention_listed(const void *q, const void *k_ctx, const void *v_c
  * queries at rows b*width .. b*width + width - 1, right padding computed like any other position).
  * K / V caches: element strides stride_row / stride_head / stride_pos, cache_len >= width positions.
  * bf16, head_dim 128, 256 or 512, contiguous key rows (stride_pos == head_dim); fp32 accumulation.  No workspace.
- * One workgroup of 8 waves per query block.  Head dim 128: 256 queries, four pairs of a score wave and a value wave;
- * 512: 64 queries, four score waves and four value waves, in chains of blocks when a launch has more than two rounds
- * of them; 256: 192 queries, each wave one 128-dimension slice, partial scores added through LDS.
+ * Head dim 128: a workgroup of 8 waves per 256 queries, four pairs of a score wave and a value wave, or of 4 waves per
+ * 192 queries where that takes fewer rounds; 512: 8 waves per 64 queries, four score waves and four value waves, in
+ * chains of blocks where a launch has two rounds of them or more and chains are predicted to end first (the rules and
+ * what they measured are beside the kernels); 256: 8 waves per 192 queries, each one 128-dimension slice, partial scores
+ * added through LDS.
  */
 int omni_prefill_attention(const void *q, const void *k_cache, const void *v_cache, int64_t stride_row,
                            int64_t stride_head, int64_t stride_pos, int64_t cache_len, int64_t cache_rows,

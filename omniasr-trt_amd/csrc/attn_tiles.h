@@ -71,8 +71,8 @@ __device__ __forceinline__ void load_tile_clamped(KVTile<D>& t, const char* kt, 
 // same in K and V; otherwise the tile is load_tile_clamped's (``rows`` is read all the same, any 32 entries).  Only
 // addresses are selected, so one set of loads serves both kinds: with the two kinds' loads under a branch the wait at
 // its join covers every load in flight, and the next tile's loads no longer overlap this tile's math (measured, the
-// beams' attention of 12 layers at 8 inputs x 5 beams, 64 generated keys: 704 -> 680 us at 8 heads x 512, 686 -> 669 at
-// 32 x 128; 2 inputs, 3 generated keys: 265 -> 254 us).
+// beams' attention of 12 layers at 8 inputs x 5 beams, 64 generated keys over contexts of 800-1900: 559 -> 539 us at 8
+// heads x 512, 490 -> 476 at 32 x 128; contexts of 250-300: 273 -> 255 and 273 -> 258 us).
 template <int D, uint32_t kRow = D * 2>
 __device__ __forceinline__ void load_tile_either(KVTile<D>& t, const char* kt, const char* vt, bool gathered,
                                                  const uint32_t* rows, int kmax, int vstop, int c, int g) {

@@ -15,9 +15,9 @@
 // per row spreads the group's reads over N CUs): the row's max and sum are two workgroup reductions in a fixed order;
 // each offer's value becomes a 32-bit number ordered as the choice is.  The N-th largest of a wave's threads' bests is a
 // floor under the row's N best, so only the offers at or above the largest floor (few more than N) become 64-bit keys,
-// value above inverted index, and wave 0 ranks them by counting.  What bounds it is that chain at one row's size, not
-// the 20 KB: as N rounds of a 64-bit scan of all offers and a wave-wide maximum, at three levels, the launch took 18 us (now 11)
-// at 8 groups x 5 beams x 10288; those rounds remain for rows with more than 256 offers at the floor (equal values).
+// value above inverted index, and wave 0 ranks them by counting.  What bounds it is that chain at one row's size, not the
+// 20 KB: as N rounds of a 64-bit scan of all offers and a wave-wide maximum, at three levels, the launch took 18 us (now
+// 11) at 8 groups x 5 beams x 10288; those rounds remain for rows with more than 256 offers at the floor (equal values).
 // The row writes them through to the device's coherence point (the rows of a group run on different XCDs, whose L2s
 // are not coherent) and takes the group's ticket; the last row of the group reads the N rows' lists and merges them
 // into the group's N best.  Every selection is by (value, index), so the result does not depend on which row

@@ -309,13 +309,14 @@ __global__ __launch_bounds__(64 * kPwWaves) __attribute__((amdgpu_waves_per_eu(2
 //    two more barriers (uniform over the workgroup: a flag every wave reads after the tile's barrier).
 //
 // What bounds a tile (64 queries x 64 keys): 2048 clocks of matrix work per SIMD, 2048 of the CU's vector memory path
-// (128 KB of K and V at 64 bytes a clock), 1860 of LDS; a tile takes ~3000, as a value wave issues its loads and its
-// products in one order.  The kernel this replaced added the partial scores of four 128-dimension slices through LDS,
-// with three barriers per 32 keys of 96 queries (5500 clocks for 1536 of matrix work).  Measured, 8 heads: 8 contexts
-// x 2048 521 -> 357 us (770 TFLOP/s; in chains 334, see ws_group); one context of 1433, where the longest block is the launch, 110 -> 39 us.  Tried:
-// 8-byte V loads of the operand's own rows, 390 / 45 us (the memory path takes a load instruction per 64 lanes, not
-// only its bytes); the loads spread between the products, 390-430 us (the tile's rows arrive later and its products
-// compete with the scores'); K rows brought by the score waves, 404 us; wave priorities, no change.
+// (128 KB of K and V at 64 bytes a clock), 1860 of LDS; as a value wave issues its loads and its products in one order, a
+// tile takes ~3000 (1.3 us) where one context leaves CUs idle, and ~5200 (2.5 us, 39% of it matrix work) with every CU
+// reading its XCD's L2.  The kernel this replaced added the partial scores of four 128-dimension slices through LDS, with
+// three barriers per 32 keys of 96 queries (5500 clocks for 1536 of matrix work).  Measured, 8 heads: 8 contexts x 2048
+// 521 -> 357 us (770 TFLOP/s; in chains 329, see ws_group); one context of 1433, where the longest block is the launch,
+// 110 -> 38 us.  Tried: 8-byte V loads of the operand's own rows, 390 / 45 us (the memory path takes a load instruction
+// per 64 lanes, not only its bytes); the loads spread between the products, 390-430 us (the tile's rows arrive later and
+// its products compete with the scores'); K rows brought by the score waves, 404 us; wave priorities, no change.
 constexpr int kWsD = 512, kWsQ = 64, kWsK = 64;
 constexpr int kWsRow = kWsD * 2 + 16;  // LDS bytes per K row
 constexpr int kWsAhead = 4;
@@ -371,11 +372,11 @@ inline int ws_longest(int nqb, int units8, int group) {
 //    units, 225 with 8, 253 with 16), and 2% for a unit alone (8 x 2048 336, with 2 330).
 // Below two rounds nothing evens out (2 contexts x 1433, 1.4 rounds: 49.5 us in chains, 47.9 without), nor with one unit,
 // whose longest block is the launch (1 x 4100: 152, 146).
-// Measured at 103 shapes, 8 heads, 2 to 16 contexts x 330 to 3000, every group size: the choice is within 1% of the best
-// one on the mean, 14% at most (16 x 640, 126 us against 111).  us, 8 contexts x width, without chains / in the chosen
-// groups: 500 42 / 37, 1984 317 (none chosen; 343 with all 8), 2048 360 / 330, 2049 369 / 354, 2300 432 / 398, 2560 507 /
-// 488, 3000 640 (none); 5 x 1024 84 / 74; 12 x 500 78 / 64; 16 x 1536 443 / 391.  The choice takes the host ~2 ns for each
-// block of each candidate.
+// Measured at 103 shapes, 8 heads, 2 to 16 contexts x 330 to 3000, every group size, repeated on one state: the choice is
+// within 1% of the best one on the mean, 14% at most (16 x 640, 126 us against 111).  us, 8 contexts x width, without
+// chains / in the chosen groups: 500 42 / 37, 1984 317 (none chosen; 343 with all 8), 2048 360 / 330, 2049 369 / 354, 2300
+// 432 / 398, 2560 507 / 488, 3000 640 (none); 5 x 1024 84 / 74; 12 x 500 78 / 64; 16 x 1536 443 / 391.  The choice takes
+// the host ~2 ns for each block of each candidate.
 inline int ws_group(int nqb, int units8) {
   if ((int64_t)nqb * units8 < 2 * kWsPerXcd || units8 < 2) return 0;
   const float n = (float)nqb;

@@ -296,7 +296,7 @@ __device__ __forceinline__ void merge_batches(const AttnArgs& a, int b, int h, i
 
 // A batch is kS partials x kR x 256 floats, one memory round trip (~2 us at the coherence point) each: with few queries
 // a batch holds more partials, so the 32 splits of a lone row at 8 heads x 512 are one round trip instead of four
-// (one query over 1433 keys: 17.0 -> 13.1 us).
+// (one query over 1433 keys, by itself: 17.0 -> 13.1 us with all 32 at work).
 template <typename OutT>
 __device__ void merge_splits_fast(const AttnArgs& a, int b, int h, int nact, int d0 = 0, int dw = -1,
                                   int64_t first_slot = -1, int64_t gen_slot = -1) {

@@ -193,7 +193,7 @@ def test_verify_attention_wide_heads_up_to_32_queries(cuda, t, d):
 def test_prefill_attention(cuda, width, d, b, h):
     """Causal attention over whole contexts (src/omniasr_trt/decode.py:163-164) against the oracle's verify attention
     with query p of a context over keys [0, p]: cache rows addressed through slots, widths that are not multiples
-    of the query block (256 queries at head dim 128, 192 at 256, 64 at 512) or of the key tile; heads x contexts a
+    of the query block (256 or 192 queries at head dim 128, 192 at 256, 64 at 512) or of the key tile; heads x contexts a
     multiple of 8 (the XCD-ordered workgroup map) or not (the plain one); at head dim 128 also widths past one
     block and up to five blocks."""
     g = gen(60 + width)
@@ -688,8 +688,9 @@ def test_verify_attention_f32_mfma(cuda, d, h, t, rows, separate):
 @pytest.mark.parametrize("grow", [0.0, 40.0])
 def test_prefill_attention_512(cuda, width, b, h, grow):
     """The head-dim 512 prefill at the edges of its 64-query blocks and 64-key tiles, one to six tiles.  The last four
-    shapes: chains of two or more blocks per workgroup, 72, 66, 64 and 80 blocks over 32 workgroups, in one group of units
-    and in groups of two (the last of one).  ``grow``: scores that climb along the context by far more than the softmax reference's guard, so that it moves on later tiles too.
+    shapes: chains of two or more blocks per workgroup, 72, 66, 64 and 80 blocks over 32 workgroups, in one group of all
+    units and in groups of two.  ``grow``: scores that climb along the context by far more than the softmax reference's
+    guard, so that it moves on later tiles too.
     Cache rows past the context hold NaN (stale memory): nothing of them may reach the output."""
     g = gen(512 + width + b)
     rows, cap, d = 4, -(-width // 64) * 64 + 32, 512
